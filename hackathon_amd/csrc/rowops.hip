@@ -13,8 +13,13 @@ namespace {
 
 // Row held in registers: thread t owns columns t + 256*i (i < V), loaded
 // together (clamped, masked) before any reduction, so a row costs one load
-// latency instead of one per 256 columns and pass. Per-thread partial sums
-// run in increasing column order, then the block sum.
+// latency instead of one per 256 columns and pass. The kernels load their
+// weight rows the same way, ahead of the reductions: a layer's weights are
+// read once per tick and come from HBM, and a load left behind a reduction
+// adds its whole latency to a kernel that is little else (one row, MI355X,
+// in the tick, us before and after: rms_ln 12.6, 5.6; ln_res_rms 11.7, 5.1;
+// rmsnorm 6.2, 4.4; mamba2_post 18.4, 8.3; slstm_post 8.8, 7.3).
+// Per-thread partial sums run in increasing column order, then the block sum.
 template <int V>
 struct RowRegs {
   float v[V];
@@ -54,15 +59,16 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ 
                                                       int64_t ldl) {
   __shared__ float red[4];
   const int64_t row = blockIdx.x;
-  RowRegs<V> r;
+  RowRegs<V> r, wr;
   r.load(x + row * ldx, width);
+  wr.load(w, width);
   const float ss = block_sum(r.sumsq(width, 0.0f), red);
   const float inv = 1.0f / sqrtf(ss / (float)width + eps);
 #pragma unroll
   for (int i = 0; i < V; ++i) {
     const int c = threadIdx.x + 256 * i;
     if (c < width) {
-      const float o = (r.v[i] * inv) * w[c];
+      const float o = (r.v[i] * inv) * wr.v[i];
       if (out) out[row * ldo + c] = o;
       if (out_lp) out_lp[row * ldl + c] = f32_to_lp_bits(o, lp_fmt);
     }
@@ -104,14 +110,16 @@ __global__ __launch_bounds__(256) void rms_ln_kernel(const float* __restrict__ x
                                                      float* __restrict__ xn) {
   __shared__ float red[4];
   const int64_t row = blockIdx.x;
-  RowRegs<V> r;
+  RowRegs<V> r, wr, wl;
   r.load(x + row * width, width);
+  wr.load(w_rms, width);
+  wl.load(w_ln, width);
   const float ss = block_sum(r.sumsq(width, 0.0f), red);
   const float inv = 1.0f / sqrtf(ss / (float)width + eps);
 #pragma unroll
   for (int i = 0; i < V; ++i) {
     const int c = threadIdx.x + 256 * i;
-    r.v[i] = c < width ? (r.v[i] * inv) * w_rms[min(c, width - 1)] : 0.0f;
+    r.v[i] = c < width ? (r.v[i] * inv) * wr.v[i] : 0.0f;
     if (c < width) {
       a[row * width + c] = r.v[i];
       if (a_lp) a_lp[row * width + c] = f32_to_lp_bits(r.v[i], lp_fmt);
@@ -122,7 +130,7 @@ __global__ __launch_bounds__(256) void rms_ln_kernel(const float* __restrict__ x
 #pragma unroll
   for (int i = 0; i < V; ++i) {
     const int c = threadIdx.x + 256 * i;
-    if (c < width) xn[row * width + c] = ((r.v[i] - mean) * rstd) * w_ln[c];
+    if (c < width) xn[row * width + c] = ((r.v[i] - mean) * rstd) * wl.v[i];
   }
 }
 
@@ -137,15 +145,17 @@ __global__ __launch_bounds__(256) void ln_res_rms_kernel(const float* __restrict
                                                          uint16_t* __restrict__ a_lp, int lp_fmt) {
   __shared__ float red[4];
   const int64_t row = blockIdx.x;
-  RowRegs<V> r, xr;
+  RowRegs<V> r, xr, wl, wr;
   r.load(y + row * width, width);
   xr.load(x + row * width, width);
+  wl.load(w_ln, width);
+  wr.load(w_rms, width);
   const float mean = block_sum(r.sum(width), red) / (float)width;
   const float rstd = 1.0f / sqrtf(block_sum(r.sumsq(width, mean), red) / (float)width + 1e-5f);
 #pragma unroll
   for (int i = 0; i < V; ++i) {
     const int c = threadIdx.x + 256 * i;
-    r.v[i] = c < width ? ((r.v[i] - mean) * rstd) * w_ln[min(c, width - 1)] + xr.v[i] : 0.0f;
+    r.v[i] = c < width ? ((r.v[i] - mean) * rstd) * wl.v[i] + xr.v[i] : 0.0f;
     if (c < width) x[row * width + c] = r.v[i];
   }
   const float ss = block_sum(r.sumsq(width, 0.0f), red);
@@ -154,7 +164,7 @@ __global__ __launch_bounds__(256) void ln_res_rms_kernel(const float* __restrict
   for (int i = 0; i < V; ++i) {
     const int c = threadIdx.x + 256 * i;
     if (c < width) {
-      const float o = (r.v[i] * inv) * w_rms[c];
+      const float o = (r.v[i] * inv) * wr.v[i];
       a[row * width + c] = o;
       if (a_lp) a_lp[row * width + c] = f32_to_lp_bits(o, lp_fmt);
     }
@@ -174,8 +184,10 @@ __global__ void stage_features_kernel(const float* __restrict__ feat, int n_rows
   }
 }
 
-// Row values held in registers (inner <= 256 * kMambaPostMax).
+// Row values held in registers, U per thread (inner <= 256 * U <= 256 *
+// kMambaPostMax); every operand is loaded before the first use.
 constexpr int kMambaPostMax = 32;
+template <int U>
 __global__ __launch_bounds__(256) void mamba2_post_kernel(
     const float* __restrict__ ssm_out, int n_parts, int64_t part_stride,
     const float* __restrict__ x, int64_t ldx, const float* __restrict__ z, int64_t ldz,
@@ -190,25 +202,34 @@ __global__ __launch_bounds__(256) void mamba2_post_kernel(
   const int64_t row = blockIdx.x;
   const float* xr = x + row * ldx;
   const float* zr = z + row * ldz;
-  float yv[kMambaPostMax];
+  float yv[U], xv[U], zv[U], dv[U], wv[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = min((int)threadIdx.x + 256 * u, inner - 1);
+    yv[u] = ssm_out[row * inner + c];
+    xv[u] = xr[c];
+    zv[u] = zr[c];
+    dv[u] = d[c / head_size];
+    wv[u] = w[c];
+  }
+  for (int q = 1; q < n_parts; ++q)
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      yv[u] += ssm_out[row * inner + min((int)threadIdx.x + 256 * u, inner - 1) + q * part_stride];
   float ss = 0.0f;
 #pragma unroll
-  for (int u = 0; u < kMambaPostMax; ++u) {
-    const int c = threadIdx.x + 256 * u;
-    yv[u] = 0.0f;
-    if (c < inner) {
-      const float so = plane_sum(ssm_out, row * inner + c, n_parts, part_stride);
-      yv[u] = (so + d[c / head_size] * xr[c]) * silu(zr[c]);
-      ss += yv[u] * yv[u];
-    }
+  for (int u = 0; u < U; ++u) {
+    const bool live = (int)threadIdx.x + 256 * u < inner;
+    yv[u] = live ? (yv[u] + dv[u] * xv[u]) * silu(zv[u]) : 0.0f;
+    if (live) ss += yv[u] * yv[u];
   }
   ss = block_sum(ss, red);
   const float inv = 1.0f / sqrtf(ss / (float)inner + 1e-5f);
 #pragma unroll
-  for (int u = 0; u < kMambaPostMax; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int c = threadIdx.x + 256 * u;
     if (c < inner) {
-      const float o = (yv[u] * inv) * w[c];
+      const float o = (yv[u] * inv) * wv[u];
       if (out) out[row * inner + c] = o;
       if (out_lp) out_lp[row * inner + c] = f32_to_lp_bits(o, lp_fmt);
     }
@@ -217,7 +238,9 @@ __global__ __launch_bounds__(256) void mamba2_post_kernel(
 
 // One wave per head.
 // A head's values held in registers (head_size <= 64 * kHeadPostMax).
+// U values per lane (head_size <= 64 U).
 constexpr int kHeadPostMax = 16;
+template <int U>
 __global__ void retnet_post_kernel(const float* __restrict__ o, int n_parts, int64_t part_stride,
                                    const float* __restrict__ g, int64_t ldg, int hidden,
                                    int head_size, float* __restrict__ out,
@@ -236,28 +259,35 @@ __global__ void retnet_post_kernel(const float* __restrict__ o, int n_parts, int
   const int lane = threadIdx.x & 63;
   const int64_t ob = row * hidden + (int64_t)head * head_size;
   const float* grow = g + row * ldg + (int64_t)head * head_size;
-  float ov[kHeadPostMax];
+  float ov[U], gv[U];
   float ss = 0.0f;
 #pragma unroll
-  for (int u = 0; u < kHeadPostMax; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int j = lane + 64 * u;
     ov[u] = j < head_size ? plane_sum(o, ob + j, n_parts, part_stride) : 0.0f;
-    ss += ov[u] * ov[u];
+    gv[u] = j < head_size ? grow[j] : 0.0f;
   }
+#pragma unroll
+  for (int u = 0; u < U; ++u) ss += ov[u] * ov[u];
   ss = wave_sum(ss);
   const float inv = 1.0f / sqrtf(ss / (float)head_size + 1e-6f);
 #pragma unroll
-  for (int u = 0; u < kHeadPostMax; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int j = lane + 64 * u;
     if (j < head_size) {
-      const float v = silu(grow[j]) * (ov[u] * inv);
+      const float v = silu(gv[u]) * (ov[u] * inv);
       if (out) out[ob + j] = v;
       if (out_lp) out_lp[ob + j] = f32_to_lp_bits(v, lp_fmt);
     }
   }
 }
 
-// One wave per group, then a block-wide LayerNorm over the whole row.
+// One wave per group (gsize <= 64 U), then a block-wide LayerNorm over the
+// whole row. The row, the skip row and every weight are loaded together
+// before the first reduction, and the row stays in registers through both
+// norms.
+constexpr int kGroupPostMax = 16;
+template <int U>
 __global__ void slstm_post_kernel(const float* __restrict__ y, const float* __restrict__ skip,
                                   const float* __restrict__ gn_w, const float* __restrict__ gn_b,
                                   const float* __restrict__ ln_w, int hidden, int gsize,
@@ -268,41 +298,54 @@ __global__ void slstm_post_kernel(const float* __restrict__ y, const float* __re
   const int grp = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
   const int64_t base = row * hidden + (int64_t)grp * gsize;
+  const int c0 = grp * gsize;
+  float v[U], sk[U], gw[U], gb[U], lw[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int j = min(lane + 64 * u, gsize - 1);
+    v[u] = y[base + j];
+    sk[u] = skip[base + j];
+    gw[u] = gn_w[c0 + j];
+    gb[u] = gn_b[c0 + j];
+    lw[u] = ln_w[c0 + j];
+  }
   float s = 0.0f;
-#pragma unroll 8
-  for (int j = lane; j < gsize; j += 64) s += y[base + j];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (lane + 64 * u < gsize) s += v[u];
   const float mean = wave_sum(s) / (float)gsize;
-  float v = 0.0f;
-#pragma unroll 8
-  for (int j = lane; j < gsize; j += 64) {
-    const float dlt = y[base + j] - mean;
-    v += dlt * dlt;
-  }
-  const float rstd = 1.0f / sqrtf(wave_sum(v) / (float)gsize + 1e-5f);
+  float q = 0.0f;
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (lane + 64 * u < gsize) {
+      const float dlt = v[u] - mean;
+      q += dlt * dlt;
+    }
+  const float rstd = 1.0f / sqrtf(wave_sum(q) / (float)gsize + 1e-5f);
   float rs = 0.0f;
-#pragma unroll 8
-  for (int j = lane; j < gsize; j += 64) {
-    const int c = grp * gsize + j;
-    const float o = ((y[base + j] - mean) * rstd) * gn_w[c] + gn_b[c] + skip[base + j];
-    x1[base + j] = o;
-    rs += o;
-  }
-  __threadfence_block();
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (lane + 64 * u < gsize) {
+      v[u] = ((v[u] - mean) * rstd) * gw[u] + gb[u] + sk[u];
+      x1[base + lane + 64 * u] = v[u];
+      rs += v[u];
+    }
   const float rmean = block_sum(rs, red) / (float)hidden;
   float rv = 0.0f;
-#pragma unroll 8
-  for (int j = lane; j < gsize; j += 64) {
-    const float dlt = x1[base + j] - rmean;
-    rv += dlt * dlt;
-  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (lane + 64 * u < gsize) {
+      const float dlt = v[u] - rmean;
+      rv += dlt * dlt;
+    }
   const float rrstd = 1.0f / sqrtf(block_sum(rv, red) / (float)hidden + 1e-5f);
-#pragma unroll 8
-  for (int j = lane; j < gsize; j += 64) {
-    const int c = grp * gsize + j;
-    const float o = ((x1[base + j] - rmean) * rrstd) * ln_w[c];
-    if (xn) xn[base + j] = o;
-    if (xn_lp) xn_lp[base + j] = f32_to_lp_bits(o, lp_fmt);
-  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (lane + 64 * u < gsize) {
+      const float o = ((v[u] - rmean) * rrstd) * lw[u];
+      if (xn) xn[base + lane + 64 * u] = o;
+      if (xn_lp) xn_lp[base + lane + 64 * u] = f32_to_lp_bits(o, lp_fmt);
+    }
 }
 
 // One wave per head (= GroupNorm group); U values per lane (head size <=
@@ -445,7 +488,9 @@ __global__ void mlstm_qkv_kernel(const float* __restrict__ x_conv, const float* 
 // block's tail), of q, k and v with 16-byte loads, stores them, and
 // accumulates their NOUT gate-row products; the work-group's NOUT sums (in
 // a fixed order) are segment seg's partial pre-activations, plane seg of
-// if_part [segs][n_rows][NOUT]; plane 0 also carries the bias.
+// if_part [segs][n_rows][n_out]; plane 0 also carries the bias. With
+// gridDim.z > 1 the n_out gate rows are dealt out NOUT to a work-group, each
+// computing the same q, k and v (z 0 stores them).
 template <int NOUT, int R>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void mlstm_qkv_if_kernel(
     ConvIn conv, const float* __restrict__ x_m, int64_t ld_xm,
@@ -456,6 +501,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   static_assert(R * NOUT <= 64, "one butterfly for all sums");
   __shared__ float red[4][R * NOUT];
   const int seg = blockIdx.x;
+  const int out0 = blockIdx.z * NOUT;      // first gate row
+  const int n_out = gridDim.z * NOUT;
+  const bool first = blockIdx.z == 0;
+  w_if += (int64_t)out0 * 3 * inner;
   const int rbase = blockIdx.y * R;  // rows rbase .. rbase + R - 1 (past n_rows: the last row)
   const int tid = threadIdx.x;
   const int per = (inner >> 2) / gridDim.x;  // 4-column blocks per segment
@@ -509,7 +558,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
                           conv1(cb.y, cw0.y, cw1.y, cw2.y, cw3.y, s0.y, s1.y, s2.y, x0.y),
                           conv1(cb.z, cw0.z, cw1.z, cw2.z, cw3.z, s0.z, s1.z, s2.z, x0.z),
                           conv1(cb.w, cw0.w, cw1.w, cw2.w, cw3.w, s0.w, s1.w, s2.w, x0.w));
-      if (rbase + r < n_rows)
+      if (first && rbase + r < n_rows)
         reinterpret_cast<float4*>(conv.out + (int64_t)rows[r] * inner)[nb] = xc[r];
     }
     // W[nb][o][h]: block nb's 4x4 weights, row o = output column 4nb + o
@@ -526,7 +575,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
       q[r] = make_float4(dot4(xc[r], bq[0]), dot4(xc[r], bq[1]), dot4(xc[r], bq[2]), dot4(xc[r], bq[3]));
       k[r] = make_float4(dot4(xc[r], bk[0]), dot4(xc[r], bk[1]), dot4(xc[r], bk[2]), dot4(xc[r], bk[3]));
       v[r] = make_float4(dot4(xm[r], bv[0]), dot4(xm[r], bv[1]), dot4(xm[r], bv[2]), dot4(xm[r], bv[3]));
-      if (rbase + r < n_rows) {
+      if (first && rbase + r < n_rows) {
         float4* q4o = reinterpret_cast<float4*>(qkv + (int64_t)rows[r] * 3 * inner);
         q4o[nb] = q[r];
         q4o[(inner >> 2) + nb] = k[r];
@@ -554,10 +603,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   if (tid < NV) {
     const int r = tid / NOUT, n = tid % NOUT;
     if (rbase + r < n_rows) {
-      float t = seg == 0 ? b_if[n] : 0.0f;
+      float t = seg == 0 ? b_if[out0 + n] : 0.0f;
 #pragma unroll
       for (int w2 = 0; w2 < 4; ++w2) t += red[w2][tid];
-      if_part[((int64_t)seg * n_rows + rbase + r) * NOUT + n] = t;
+      if_part[((int64_t)seg * n_rows + rbase + r) * n_out + out0 + n] = t;
     }
   }
 }
@@ -659,9 +708,18 @@ int mamba2_post(const float* ssm_out, int n_parts, int64_t part_stride, const fl
   if (n_rows == 0 && lc.jobs() == 0) return HK_OK;
   HK_REQUIRE(inner <= 256 * kMambaPostMax && n_parts >= 1,
              "mamba2_post: inner %d above %d or no planes", inner, 256 * kMambaPostMax);
-  hipLaunchKernelGGL(mamba2_post_kernel, dim3(rows_and_commit(n_rows, lc, 256)), dim3(256), 0, s,
-                     ssm_out, n_parts, part_stride, x, ldx, z, ldz, d, w, inner, head_size, out,
-                     out_lp, lp_fmt, n_rows, lc);
+#define HK_POST(U)                                                                              \
+  hipLaunchKernelGGL(mamba2_post_kernel<U>, dim3(rows_and_commit(n_rows, lc, 256)), dim3(256), 0, \
+                     s, ssm_out, n_parts, part_stride, x, ldx, z, ldz, d, w, inner, head_size, out, \
+                     out_lp, lp_fmt, n_rows, lc)
+  if (inner <= 256 * 4) {
+    HK_POST(4);
+  } else if (inner <= 256 * 16) {
+    HK_POST(16);
+  } else {
+    HK_POST(kMambaPostMax);
+  }
+#undef HK_POST
   HK_LAUNCH_CHECK();
   return HK_OK;
 }
@@ -679,8 +737,15 @@ int retnet_post(const float* o, int n_parts, int64_t part_stride, const float* g
   const int threads = 64 * heads;
   const unsigned grid =
       (unsigned)(n_rows + (lc.jobs() + adv.jobs() + threads - 1) / threads);
-  hipLaunchKernelGGL(retnet_post_kernel, dim3(grid), dim3(threads), 0, s, o, n_parts, part_stride,
-                     g, ldg, hidden, head_size, out, out_lp, lp_fmt, n_rows, lc, adv);
+#define HK_POST(U)                                                                             \
+  hipLaunchKernelGGL(retnet_post_kernel<U>, dim3(grid), dim3(threads), 0, s, o, n_parts, part_stride, \
+                     g, ldg, hidden, head_size, out, out_lp, lp_fmt, n_rows, lc, adv)
+  if (head_size <= 64 * 4) {
+    HK_POST(4);
+  } else {
+    HK_POST(kHeadPostMax);
+  }
+#undef HK_POST
   HK_LAUNCH_CHECK();
   return HK_OK;
 }
@@ -691,8 +756,20 @@ int slstm_post(const float* y, const float* skip, const float* gn_w, const float
   if (n_rows == 0) return HK_OK;
   HK_REQUIRE(groups >= 1 && groups <= 16 && hidden % groups == 0,
              "slstm_post: %d groups unsupported", groups);
-  hipLaunchKernelGGL(slstm_post_kernel, dim3(n_rows), dim3(64 * groups), 0, s, y, skip, gn_w,
-                     gn_b, ln_w, hidden, hidden / groups, x1, xn, xn_lp, lp_fmt);
+  const int gsize = hidden / groups;
+  HK_REQUIRE(gsize <= 64 * kGroupPostMax, "slstm_post: group of %d above %d", gsize,
+             64 * kGroupPostMax);
+#define HK_POST(U)                                                                            \
+  hipLaunchKernelGGL(slstm_post_kernel<U>, dim3(n_rows), dim3(64 * groups), 0, s, y, skip, gn_w, \
+                     gn_b, ln_w, hidden, gsize, x1, xn, xn_lp, lp_fmt)
+  if (gsize <= 64 * 2) {
+    HK_POST(2);
+  } else if (gsize <= 64 * 8) {
+    HK_POST(8);
+  } else {
+    HK_POST(kGroupPostMax);
+  }
+#undef HK_POST
   HK_LAUNCH_CHECK();
   return HK_OK;
 }
@@ -776,15 +853,25 @@ int mlstm_qkv_if(const ConvIn& conv, const float* x_m, int64_t ld_xm, const floa
              "mlstm_qkv_if: inner %d, %d gate rows, %d segments or alignment unsupported", inner,
              n_out, segs);
   // R rows per work-group share each block's weight loads (R * n_out <= 64).
+  // Sixteen gate rows of few request rows go four to a work-group: one
+  // work-group reads 12 KB of gate weights per 4-column block and would take
+  // a segment's 196 KB through one CU (one row: 14.4 us, dealt out 10.5). From 64
+  // rows up (64 work-groups) the repeated q, k, v products cost more.
   const dim3 block(256);
 #define HK_QKV_IF(NOUT, R)                                                                      \
-  hipLaunchKernelGGL((mlstm_qkv_if_kernel<NOUT, R>), dim3(segs, (n_rows + (R)-1) / (R)), block, \
+  hipLaunchKernelGGL((mlstm_qkv_if_kernel<NOUT, R>), dim3(segs, (n_rows + (R)-1) / (R), n_out / (NOUT)), block, \
                      0, s, conv, x_m, ld_xm, wq, wk, wv, n_rows, inner, k_div, w_if, b_if, qkv, \
                      ks, if_part)
   switch (n_out) {
     case 4: HK_QKV_IF(4, 4); break;
     case 8: HK_QKV_IF(8, 4); break;
-    case 16: HK_QKV_IF(16, 4); break;
+    case 16:
+      if (n_rows < 64) {
+        HK_QKV_IF(4, 4);
+      } else {
+        HK_QKV_IF(16, 4);
+      }
+      break;
     default: HK_QKV_IF(32, 2); break;
   }
 #undef HK_QKV_IF

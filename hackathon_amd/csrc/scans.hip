@@ -872,7 +872,7 @@ __global__ __launch_bounds__(64 * NWV) void mlstm_gates_kernel(
     for (int p = 1; p < n_parts; ++p) g += gp[p * part_stride];
   };
   fill(rq[0], rk[0], rg[0], 0);
-  fill(rq[1], rk[1], rg[1], B);
+  if (len > B) fill(rq[1], rk[1], rg[1], B);  // (a short run reads one block)
 
   auto block = [&](const float (&q)[B][PER], const float (&k)[B][PER], float g, int tb, int par) {
     float ig[B], fg[B], em[B];
