@@ -428,8 +428,11 @@ struct Engine {
   // back to the caller's stream per tick (all streams at default priority).
   // Four streams in all, one per hardware queue of a default HIP process:
   // the caller's stream runs the xLSTM tower's first run group (the longest
-  // runs), side[0] its second group, side[1] Mamba2, side[2] RetNet then
-  // Hawk.
+  // runs), side[0] its second group, side[1] Mamba2, side[2] RetNet and
+  // Hawk; a tick without a second group runs Hawk on side[0] (RetNet and
+  // Hawk together are 42 of a two-layer tick's launches against the xLSTM's
+  // 32, and a small tick is the longest stream's chain of launches:
+  // 8 of 64 rows 642 us on one stream, 547 on two).
   static constexpr int kSide = 3;
   hipStream_t side[kSide] = {nullptr, nullptr, nullptr};
   // hipGraph replay of small ticks (the reference captures its whole step
@@ -1109,7 +1112,7 @@ int tower_tail(Engine& e, int t, TowerWS& w, const Group& g, float* preds, hipSt
 
 // Every tower of the tick, enqueued layer by layer: the xLSTM on the caller's
 // stream s (run group g1) and, when split, side[0] (group g2); Mamba2 on
-// side[1]; RetNet and Hawk on side[2].
+// side[1]; RetNet on side[2]; Hawk on side[0], or on side[2] when split.
 // - The two xLSTM groups' persistent sLSTM launches alternate (g2 layer l
 //   after g1 layer l-1, g1 layer l after g2 layer l), so two persistent
 //   launches never compete for co-residency.
@@ -1120,9 +1123,10 @@ int run_towers(Engine& e, const Group& all, const Group& g1, const Group* g2, hi
                      float* preds) {
   TowerWS& w1 = e.ws[kXLSTM];
   TowerWS& w2 = e.ws_x2;
+  const hipStream_t hs = g2 ? e.side[2] : e.side[0];  // Hawk's (see retnet_stream)
   HK_TRY(tower_head(e, kMamba2, e.ws[kMamba2], all, e.side[1]));
   HK_TRY(tower_head(e, kRetNet, e.ws[kRetNet], all, e.side[2]));
-  HK_TRY(tower_head(e, kHawk, e.ws[kHawk], all, e.side[2]));
+  HK_TRY(tower_head(e, kHawk, e.ws[kHawk], all, hs));
   HK_TRY(tower_head(e, kXLSTM, w1, g1, s));
   if (g2) HK_TRY(tower_head(e, kXLSTM, w2, *g2, e.side[0]));
   for (int l = 0; l < e.d.D; ++l) {
@@ -1139,11 +1143,11 @@ int run_towers(Engine& e, const Group& all, const Group& g1, const Group* g2, hi
     }
     HK_TRY(tower_layer(e, kMamba2, e.ws[kMamba2], all, l, nullptr, SlOrder{}, e.side[1]));
     HK_TRY(tower_layer(e, kRetNet, e.ws[kRetNet], all, l, nullptr, SlOrder{}, e.side[2]));
-    HK_TRY(tower_layer(e, kHawk, e.ws[kHawk], all, l, nullptr, SlOrder{}, e.side[2]));
+    HK_TRY(tower_layer(e, kHawk, e.ws[kHawk], all, l, nullptr, SlOrder{}, hs));
   }
   HK_TRY(tower_tail(e, kMamba2, e.ws[kMamba2], all, preds, e.side[1]));
   HK_TRY(tower_tail(e, kRetNet, e.ws[kRetNet], all, preds, e.side[2]));
-  HK_TRY(tower_tail(e, kHawk, e.ws[kHawk], all, preds, e.side[2]));
+  HK_TRY(tower_tail(e, kHawk, e.ws[kHawk], all, preds, hs));
   HK_TRY(tower_tail(e, kXLSTM, w1, g1, preds, s));
   if (g2) HK_TRY(tower_tail(e, kXLSTM, w2, *g2, preds, e.side[0]));
   return HK_OK;
@@ -1166,16 +1170,24 @@ int mamba2_stream(Engine& e, const Group& all, float* preds) {
   return tower_tail(e, kMamba2, w, all, preds, s);
 }
 
-// RetNet and Hawk, layer by layer, on side[2].
-int retnet_hawk_stream(Engine& e, const Group& all, float* preds) {
+// RetNet on side[2]; Hawk on side[0] when that stream has no second xLSTM
+// group, else behind RetNet, layer by layer.
+int retnet_stream(Engine& e, const Group& all, float* preds, bool hawk) {
   hipStream_t s = e.side[2];
   HK_TRY(tower_head(e, kRetNet, e.ws[kRetNet], all, s));
-  HK_TRY(tower_head(e, kHawk, e.ws[kHawk], all, s));
+  if (hawk) HK_TRY(tower_head(e, kHawk, e.ws[kHawk], all, s));
   for (int l = 0; l < e.d.D; ++l) {
     HK_TRY(tower_layer(e, kRetNet, e.ws[kRetNet], all, l, nullptr, SlOrder{}, s));
-    HK_TRY(tower_layer(e, kHawk, e.ws[kHawk], all, l, nullptr, SlOrder{}, s));
+    if (hawk) HK_TRY(tower_layer(e, kHawk, e.ws[kHawk], all, l, nullptr, SlOrder{}, s));
   }
   HK_TRY(tower_tail(e, kRetNet, e.ws[kRetNet], all, preds, s));
+  return hawk ? tower_tail(e, kHawk, e.ws[kHawk], all, preds, s) : HK_OK;
+}
+int hawk_stream(Engine& e, const Group& all, float* preds) {
+  hipStream_t s = e.side[0];
+  HK_TRY(tower_head(e, kHawk, e.ws[kHawk], all, s));
+  for (int l = 0; l < e.d.D; ++l)
+    HK_TRY(tower_layer(e, kHawk, e.ws[kHawk], all, l, nullptr, SlOrder{}, s));
   return tower_tail(e, kHawk, e.ws[kHawk], all, preds, s);
 }
 
@@ -1195,9 +1207,12 @@ int run_towers_mt(Engine& e, const Group& all, const Group& g1, const Group* g2,
     }
   }
   EnqueuePool& p = *e.pool;
-  if (g2) p.post(0, [&] { return xlstm_stream(e, e.ws_x2, *g2, e.d_xch2, preds, e.side[0]); });
+  if (g2)
+    p.post(0, [&] { return xlstm_stream(e, e.ws_x2, *g2, e.d_xch2, preds, e.side[0]); });
+  else
+    p.post(0, [&] { return hawk_stream(e, all, preds); });
   p.post(1, [&] { return mamba2_stream(e, all, preds); });
-  p.post(2, [&] { return retnet_hawk_stream(e, all, preds); });
+  p.post(2, [&] { return retnet_stream(e, all, preds, g2 != nullptr); });
   const int st = xlstm_stream(e, e.ws[kXLSTM], g1, e.d_xch, preds, s);
   std::string err;
   const int wst = p.wait(&err);  // the threads use e, all, g1, g2 until here
