@@ -1230,10 +1230,18 @@ int run_towers_mt(Engine& e, const Group& all, const Group& g1, const Group* g2,
 // cost. (Four one-request symbols in fp32 (C1): unsplit 23 us against 13 +
 // 41 split, measured 3.90 against 4.10 ms per step; 256 Zipf requests in
 // bf16 (C4): about 1000 against 500 + 24.)
+// The second group also takes the stream that Hawk would have, so it has to
+// shorten a long chain of sLSTM steps: ticks whose longest run is below
+// kSplitMinLen stay whole. Two-layer ticks, us split / whole: 32, 64 and 256
+// single requests 685 / 637, 888 / 873 and 2349 / 2285; 256 with runs of up
+// to about six 2011 / 1968; 64 single requests in fp32 1309 / 1167; with a
+// run of about fifty 256 requests 1500 / 1574 and 800 3347 / 3629.
+constexpr int kSplitMinLen = 16;
 int xlstm_split_point(const int* run_off, int n_runs, double weight_us) {
   constexpr double kStepUs = 3.0, kSymbolUs = 5.0, kGain = 0.8;
   if (n_runs < 2) return n_runs;
   const int len0 = run_off[1] - run_off[0];
+  if (len0 < kSplitMinLen) return n_runs;
   const double whole = kStepUs * len0 + kSymbolUs * n_runs;
   double best = whole;
   int best_k = n_runs;
