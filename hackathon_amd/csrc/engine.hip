@@ -1683,6 +1683,39 @@ int hk_engine_state_copy(void* h, int tower, int layer, int leaf, int slot0, int
   return HK_OK;
 }
 
+// Copies the state of slots [src0, src0 + nslots) to [dst0, dst0 + nslots)
+// (disjoint ranges): every leaf of every block, with the write-back logs as
+// they are, so the source is only read and each stored byte moves once (one
+// launch per block). Stream-ordered.
+int hk_engine_copy_slots(void* h, int src0, int dst0, int nslots, void* stream) {
+  HK_REQUIRE(h, "hk_engine_copy_slots: null handle");
+  Engine& e = *static_cast<Engine*>(h);
+  HK_REQUIRE(nslots >= 0 && src0 >= 0 && dst0 >= 0 && nslots <= e.capacity &&
+                 std::max(src0, dst0) <= e.capacity - nslots,
+             "hk_engine_copy_slots: slots out of range");
+  HK_REQUIRE(src0 + nslots <= dst0 || dst0 + nslots <= src0, "hk_engine_copy_slots: ranges overlap");
+  if (nslots == 0) return HK_OK;
+  hipStream_t s = (hipStream_t)stream;
+  for (int t = 0; t < hk::kTowers; ++t) {
+    for (int l = 0; l < e.d.D; ++l) {
+      hk::CopyList c;
+      auto add = [&](float* base, int64_t per) {
+        if (base) c.add(base + src0 * per, base + dst0 * per, nslots * per);
+      };
+      for (size_t leaf = 0; leaf < e.leaf_elems[t].size(); ++leaf)
+        add(e.state[t][l][leaf], e.leaf_elems[t][leaf]);
+      if (hk::matrix_leaf(t) >= 0) {
+        const hk::MatScanDesc m = hk::mat_state_desc(e, t, l);
+        add(m.log_hdr, (int64_t)m.heads * hk::kLogHdr);
+        add(m.log_b, (int64_t)m.heads * m.log_cap * m.rows);
+        add(m.log_g, (int64_t)m.heads * m.log_cap * m.cols);
+      }
+      HK_TRY(hk::copy_list(c, s));
+    }
+  }
+  return HK_OK;
+}
+
 // Resets slots to the reference's init_state values (zeros; the sLSTM
 // running max starts at -inf, model/xlstm.py:375). n < 0 resets every slot.
 int hk_engine_reset_slots(void* h, const int* slots_host, int n, void* stream) {

@@ -156,6 +156,18 @@ int mlstm_qkv_if(const ConvIn& conv, const float* x_m, int64_t ld_xm, const floa
 int to_lp(const float* src, uint16_t* dst, int64_t n, int lp_fmt, hipStream_t s);
 // v[i] = v[i] rounded through the 16-bit format lp_fmt, in place.
 int round_lp_inplace(float* v, int64_t n, int lp_fmt, hipStream_t s);
+// Up to kMax device arrays copied in one launch (sources and destinations
+// disjoint, fp32, 4-byte aligned).
+struct CopyList {
+  static constexpr int kMax = 16;
+  const float* src[kMax] = {};
+  float* dst[kMax] = {};
+  int64_t n[kMax] = {};      // floats
+  int64_t block0[kMax + 1] = {};  // first work-group of each array
+  int count = 0;
+  void add(const float* s, float* d, int64_t floats);
+};
+int copy_list(const CopyList& c, hipStream_t s);
 // fill with a constant
 int fill_f32(float* dst, int64_t n, float v, hipStream_t s);
 

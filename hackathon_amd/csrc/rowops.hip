@@ -624,6 +624,33 @@ __global__ void round_lp_inplace_kernel(float* __restrict__ v, int64_t n, int lp
     v[i] = round_lp(v[i], lp_fmt);
 }
 
+// Work-group i copies floats [(i - block0) * kCopyChunk, ..) of its array, 64 KB
+// in 16-byte accesses (singly where an address is not a multiple of 16, as
+// per-slot leaves of a few floats are), eight loads in flight per thread.
+constexpr int kCopyChunk = 16384;
+__global__ __launch_bounds__(256) void copy_list_kernel(CopyList c) {
+  int a = 0;
+  while (a + 1 < c.count && (int64_t)blockIdx.x >= c.block0[a + 1]) ++a;
+  const int64_t off = ((int64_t)blockIdx.x - c.block0[a]) * kCopyChunk;
+  const int n = (int)min((int64_t)kCopyChunk, c.n[a] - off);
+  const float* src = c.src[a] + off;
+  float* dst = c.dst[a] + off;
+  if ((((uintptr_t)src | (uintptr_t)dst) & 15u) != 0 || n % 4 != 0) {
+    for (int i = threadIdx.x; i < n; i += 256) gstore(dst + i, gload(src + i));
+    return;
+  }
+  const int nv = n / 4;
+  for (int i0 = threadIdx.x; i0 < nv; i0 += 256 * 8) {
+    u32x4 v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = gload16(src + 4 * min(i0 + 256 * u, nv - 1));
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (i0 + 256 * u < nv)
+        *(__attribute__((address_space(1))) u32x4*)(dst + 4 * (i0 + 256 * u)) = v[u];
+  }
+}
+
 __global__ void fill_f32_kernel(float* __restrict__ dst, int64_t n, float v) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
@@ -894,6 +921,23 @@ int to_lp(const float* src, uint16_t* dst, int64_t n, int lp_fmt, hipStream_t s)
 int round_lp_inplace(float* v, int64_t n, int lp_fmt, hipStream_t s) {
   if (n == 0) return HK_OK;
   hipLaunchKernelGGL(round_lp_inplace_kernel, dim3(grid_for(n)), dim3(256), 0, s, v, n, lp_fmt);
+  HK_LAUNCH_CHECK();
+  return HK_OK;
+}
+
+void CopyList::add(const float* s, float* d, int64_t floats) {
+  src[count] = s;
+  dst[count] = d;
+  n[count] = floats;
+  block0[count + 1] = block0[count] + (floats + kCopyChunk - 1) / kCopyChunk;
+  ++count;
+}
+
+int copy_list(const CopyList& c, hipStream_t s) {
+  const int64_t blocks = c.block0[c.count];
+  if (blocks == 0) return HK_OK;
+  HK_REQUIRE(blocks < (1LL << 31), "copy_list: too large (%lld work-groups)", (long long)blocks);
+  hipLaunchKernelGGL(copy_list_kernel, dim3((unsigned)blocks), dim3(256), 0, s, c);
   HK_LAUNCH_CHECK();
   return HK_OK;
 }

@@ -33,6 +33,7 @@ _lib.register("hk_engine_state_numel", c_int, [c_void_p, c_int, c_int, ctypes.PO
 _lib.register(
     "hk_engine_state_copy", c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p]
 )
+_lib.register("hk_engine_copy_slots", c_int, [c_void_p, c_int, c_int, c_int, c_void_p])
 _lib.register("hk_engine_reset_slots", c_int, [c_void_p, c_void_p, c_int, c_void_p])
 _lib.register("hk_engine_log_fill", c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p])
 _lib.register("hk_engine_tick", c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p])
@@ -299,14 +300,13 @@ class Engine:
     def copy_slots(self, src0: int, dst0: int, nslots: int):
         """Copy the state of slots [src0, src0+nslots) to [dst0, dst0+nslots)
         (ranges disjoint), stream-ordered: every leaf of every block, pending
-        write-back entries applied (the source's value is unchanged)."""
+        write-back entries as they are (the source is only read)."""
         assert nslots >= 0 and 0 <= src0 and 0 <= dst0
         assert max(src0, dst0) + nslots <= self.capacity
         assert src0 + nslots <= dst0 or dst0 + nslots <= src0, "slot ranges overlap"
-        for t in range(4):
-            for b in range(self.cfg.tower_depth):
-                for leaf, buf in enumerate(self._raw_leaves(t, b, src0, nslots)):
-                    self._copy_leaf(t, b, leaf, dst0, nslots, buf, True)
+        with torch.cuda.device(self.device):
+            _lib.check(_lib.lib().hk_engine_copy_slots(self._h, src0, dst0, nslots, self._stream()),
+                       "hk_engine_copy_slots")
 
     def export_state(self, slot0: int = 0, nslots: int | None = None):
         """State of slots [slot0, slot0+nslots) in the reference's init_state

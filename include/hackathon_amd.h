@@ -233,6 +233,13 @@ int hk_engine_state_numel(void* handle, int tower, int leaf, int64_t* per_slot);
 int hk_engine_state_copy(void* handle, int tower, int layer, int leaf, int slot0, int nslots,
                          void* buf, int to_engine, void* stream);
 
+/* Copies the state of slots [src0, src0+nslots) to [dst0, dst0+nslots)
+ * (disjoint ranges), every leaf of every block: the state a mask=None forward
+ * advances while the old one stays usable (model/inference_model.py:132-134).
+ * Pending write-back updates are copied as they are; the source is only
+ * read. Stream-ordered. */
+int hk_engine_copy_slots(void* handle, int src0, int dst0, int nslots, void* stream);
+
 /* Resets slots to init_state values (zeros; sLSTM running max -inf,
  * model/xlstm.py:375); n < 0 resets every slot. */
 int hk_engine_reset_slots(void* handle, const int* slots_host, int n, void* stream);
