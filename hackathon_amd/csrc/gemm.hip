@@ -495,6 +495,42 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g, float* partial, i
   }
 }
 
+// The epilogue of gemm_kernel for one fragment's lane: rows m0 .. m0 + 3 of
+// column n (batch b). Residual reads first (the residual may be the output
+// itself), then every value, then every store.
+__device__ __forceinline__ void store_f32_fragment(const GemmArgs& g, int b, int m0, int n,
+                                                   const floatx4& acc) {
+  const int M = g.M;
+  if (n >= g.N) return;
+  const GemmEpilogue& ep = g.ep;
+  const int64_t cb = (int64_t)b * g.c_bstride;
+  const float bias_v = ep.bias ? ep.bias[n + cb] : 0.0f;
+  float res[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int m = m0 + e;
+    res[e] = (ep.residual && m < M) ? ep.residual[(int64_t)m * ep.ldr + n + cb] : 0.0f;
+  }
+  float outv[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float v = acc[e] + bias_v;
+    if (ep.round_lp) v = round_lp(v, ep.lp_fmt);
+    if (ep.act == 1) v = fmaxf(v, 0.0f);
+    outv[e] = v + res[e];
+    if (ep.dt_a) outv[e] = softplus(outv[e]);
+  }
+  const int64_t nc = n + cb;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int m = m0 + e;
+    if (m >= M) continue;
+    if (ep.out) ep.out[(int64_t)m * ep.ldo + nc] = outv[e];
+    if (ep.out_lp) ep.out_lp[(int64_t)m * ep.ldl + nc] = f32_to_lp_bits(outv[e], ep.lp_fmt);
+    if (ep.dt_decay) ep.dt_decay[(int64_t)m * ep.ldd + nc] = expf(ep.dt_a[n] * outv[e]);
+  }
+}
+
 // Skinny fp32 products: at most 16 rows of A (kSkinnyRows), e.g. the fp32
 // mode's four symbols, one request each. The 64x64 tile above would stage
 // and multiply 64 rows of A per slab for these, and its split-K partial sums
@@ -575,37 +611,109 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void gemm_skinny_kernel(GemmArgs
   for (int w = 0; w < NWV - 1; ++w) acc += red[w][lane];
 
   // The fragment: lane holds rows 4*fk + e of column n0 + fr.
-  const int n = n0 + fr;
-  // The epilogue of gemm_kernel: residual reads first (the residual may be
-  // the output itself), then every value, then every store.
-  if (n >= g.N) return;
-  const GemmEpilogue& ep = g.ep;
-  const int64_t cb = (int64_t)b * g.c_bstride;
-  const float bias_v = ep.bias ? ep.bias[n + cb] : 0.0f;
-  float res[4];
+  store_f32_fragment(g, b, 4 * fk, n0 + fr, acc);
+}
+
+// BlockLinear products of more than 16 rows (fp32, K at most kBlockK): a
+// launch has few 64x64 tiles (64 rows of four 512-wide blocks: 32) and K is
+// too short to split over work-groups, so gemm_kernel left most CUs idle and
+// ran each tile's K as one chain of slabs (64 rows 14.6 us, 256 rows 15.8).
+// Here a work-group of 8 waves owns a 16 MT x 16 NT tile and all of K; the
+// waves take interleaved 16-deep k steps, kBlockU of them loaded together
+// straight into registers (A and W fragments, 16 rows x 64 bytes each), and
+// their sums meet in LDS, added in wave order, one fragment per wave. What
+// bounds it: one load latency, the products and the sum in LDS, one after the
+// other in each work-group. Measured (512-wide blocks, four of them, us, this
+// kernel / gemm_kernel): 32 rows 5.1 / 14.3, 64 6.3 / 14.4, 128 9.0 / 14.6, 256
+// 11.4 / 15.0; against float64 its error is 0.4 of gemm_kernel's (shorter
+// chains of sums). At kBlockTiles 64x64 tiles and more gemm_kernel fills the
+// device and is faster (384 rows 15.4 / 20.6, 1000 rows 26.5 / 39.8).
+constexpr int kBlockWaves = 8;
+constexpr int kBlockU = 4;
+constexpr int kBlockK = 512;
+constexpr int kBlockTiles = 192;
+
+template <int MT, int NT>
+__global__ __launch_bounds__(64 * kBlockWaves) void gemm_block_kernel(GemmArgs g, int tiles_m,
+                                                                      int tiles_n) {
+  constexpr int NWV = kBlockWaves;
+  constexpr int U = kBlockU;
+  static_assert(MT * NT <= NWV, "one fragment per wave in the sum");
+  const int nwg = gridDim.x;
+  int bid = blockIdx.x;
+  const int full = (nwg / 8) * 8;
+  if (bid < full) bid = (bid % 8) * (full / 8) + bid / 8;
+  const int tm = bid % tiles_m;
+  const int rest = bid / tiles_m;
+  const int tn = rest % tiles_n;
+  const int b = rest / tiles_n;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int fr = lane & 15;  // A row / W column of the fragments
+  const int fk = lane >> 4;  // k group: k = 16*step + 4*fk + c
+  const int m0 = tm * 16 * MT;
+  const int n0 = tn * 16 * NT;
+  const void* Asrc = (g.A2 != nullptr && b >= g.a2_from) ? g.A2 : g.A;
+  const float* Ab = static_cast<const float*>(Asrc) +
+                    (int64_t)(g.a_period > 0 ? b % g.a_period : b) * g.a_bstride + 4 * fk;
+  const float* Wb = static_cast<const float*>(g.W) + (int64_t)b * g.w_bstride + 4 * fk;
+  // rows past M and columns past N read row 0 (never stored)
+  const float* a_src[MT];
+  const float* w_src[NT];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int m = 4 * fk + e;
-    res[e] = (ep.residual && m < M) ? ep.residual[(int64_t)m * ep.ldr + n + cb] : 0.0f;
+  for (int i = 0; i < MT; ++i) {
+    const int r = m0 + 16 * i + fr;
+    a_src[i] = Ab + (int64_t)(r < g.M ? r : 0) * g.lda;
   }
-  float outv[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    float v = acc[e] + bias_v;
-    if (ep.round_lp) v = round_lp(v, ep.lp_fmt);
-    if (ep.act == 1) v = fmaxf(v, 0.0f);
-    outv[e] = v + res[e];
-    if (ep.dt_a) outv[e] = softplus(outv[e]);
+  for (int j = 0; j < NT; ++j) {
+    const int c = n0 + 16 * j + fr;
+    w_src[j] = Wb + (int64_t)(c < g.N ? c : 0) * g.ldw;
   }
-  const int64_t nc = n + cb;
+  const int ksteps = g.K / 16;
+  const int nsteps = ksteps > wave ? (ksteps - wave + NWV - 1) / NWV : 0;
+
+  floatx4 acc[MT][NT];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int m = 4 * fk + e;
-    if (m >= M) continue;
-    if (ep.out) ep.out[(int64_t)m * ep.ldo + nc] = outv[e];
-    if (ep.out_lp) ep.out_lp[(int64_t)m * ep.ldl + nc] = f32_to_lp_bits(outv[e], ep.lp_fmt);
-    if (ep.dt_decay) ep.dt_decay[(int64_t)m * ep.ldd + nc] = expf(ep.dt_a[n] * outv[e]);
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s0 = 0; s0 < nsteps; s0 += U) {
+    floatx4 av[U][MT], wv[U][NT];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // (a round past the wave's last step loads its first one again)
+      const int k = (wave + NWV * (s0 + u < nsteps ? s0 + u : 0)) * 16;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) wv[u][j] = __builtin_bit_cast(floatx4, gload16(w_src[j] + k));
+#pragma unroll
+      for (int i = 0; i < MT; ++i) av[u][i] = __builtin_bit_cast(floatx4, gload16(a_src[i] + k));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (s0 + u < nsteps) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u][i][c], wv[u][j][c], acc[i][j], 0, 0, 0);
+      }
+    }
   }
+
+  __shared__ floatx4 red[NWV][MT * NT][64];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) red[wave][i * NT + j][lane] = acc[i][j];
+  __syncthreads();
+  if (wave >= MT * NT) return;
+  floatx4 sum = red[0][wave][lane];
+#pragma unroll
+  for (int w = 1; w < NWV; ++w) sum += red[w][wave][lane];
+  store_f32_fragment(g, b, m0 + 16 * (wave / NT) + 4 * fk, n0 + 16 * (wave % NT) + fr, sum);
 }
 
 // The 16-bit CastLinear projection of at most 16 rows on packed weights:
@@ -1229,6 +1337,40 @@ int gemm_skinny(const GemmArgs& g, hipStream_t stream) {
   return HK_OK;
 }
 
+// fp32 products of more than kSkinnyRows rows with a short K (any batch
+// description).
+int gemm_block(const GemmArgs& g, hipStream_t stream) {
+  // The largest of 64x32, 64x16, 32x16 and 16x16 (rows x columns) that still
+  // gives 192 work-groups, most of the 256 CUs (asking for 320 takes smaller
+  // tiles, which read more: 256 rows 14.3 against 11.4 us).
+  static const int kTiles[4][2] = {{4, 2}, {4, 1}, {2, 1}, {1, 1}};  // (MT, NT)
+  auto tiles = [&](int c) {
+    return (int64_t)((g.M + 16 * kTiles[c][0] - 1) / (16 * kTiles[c][0])) *
+           ((g.N + 16 * kTiles[c][1] - 1) / (16 * kTiles[c][1])) * g.batch;
+  };
+  int pick = 0;
+  while (pick < 3 && tiles(pick) < 192) ++pick;
+  HK_REQUIRE(tiles(pick) < (1LL << 31), "gemm: grid too large");
+  const int mt = kTiles[pick][0], nt = kTiles[pick][1];
+  const int tiles_m = (g.M + 16 * mt - 1) / (16 * mt);
+  const int tiles_n = (g.N + 16 * nt - 1) / (16 * nt);
+  const dim3 grid((unsigned)tiles(pick)), block(64 * kBlockWaves);
+#define HK_BLOCK(MT, NT)                                                                         \
+  hipLaunchKernelGGL((gemm_block_kernel<MT, NT>), grid, block, 0, stream, g, tiles_m, tiles_n)
+  if (pick == 0) {
+    HK_BLOCK(4, 2);
+  } else if (pick == 1) {
+    HK_BLOCK(4, 1);
+  } else if (pick == 2) {
+    HK_BLOCK(2, 1);
+  } else {
+    HK_BLOCK(1, 1);
+  }
+#undef HK_BLOCK
+  HK_LAUNCH_CHECK();
+  return HK_OK;
+}
+
 }  // namespace
 
 bool packable(int N, int K) { return N > 0 && K > 0 && N % 32 == 0 && K % 64 == 0; }
@@ -1283,6 +1425,9 @@ int gemm(const GemmArgs& g, const GemmWorkspace& ws, hipStream_t stream, int spl
   const int tiles_m = (g.M + BM - 1) / BM;
   const int tiles_n = (g.N + BN - 1) / BN;
   const int64_t tiles = (int64_t)tiles_m * tiles_n * g.batch;
+  // A short K and too few 64x64 tiles to fill the device (kBlockTiles).
+  if (g.type == GemmType::kF32 && g.split_wscale == 0.0f && g.K <= kBlockK && tiles < kBlockTiles)
+    return gemm_block(g, stream);
   const int ktiles = g.K / BK;
   int splits = splits_hint;
   if (splits <= 0) {
