@@ -2,6 +2,7 @@
 // (model/kernels.py:346-401): state updated in place on active rows, idle rows
 // untouched, idle outputs zero. Shapes follow the reference's (B, n, h, k)
 // layout; every operand is a contiguous fp32 device array.
+#include <algorithm>
 #include <cstring>
 #include <string>
 
@@ -308,6 +309,23 @@ __global__ __launch_bounds__(256) void block_linear_kernel(
   out[i] = bias ? acc + bias[col] : acc;
 }
 
+// fp32 -> 16-bit (round to nearest even), eight values per thread and step:
+// two 16-byte loads, one 16-byte store. n a multiple of 8.
+template <int FMT>
+__global__ __launch_bounds__(256) void cast_rows_kernel(const float* __restrict__ x,
+                                                        uint16_t* __restrict__ out, int64_t n) {
+  const int64_t step = (int64_t)gridDim.x * 256 * 8;
+  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += step) {
+    const float4 a = gload_f4(x + i), b = gload_f4(x + i + 4);
+    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      w[j] = (uint32_t)f32_to_lp_bits_t<FMT>(v[2 * j]) | ((uint32_t)f32_to_lp_bits_t<FMT>(v[2 * j + 1]) << 16);
+    *(__attribute__((address_space(1))) u32x4*)(out + i) = u32x4{w[0], w[1], w[2], w[3]};
+  }
+}
+
 int elementwise_grid(int64_t n, unsigned* blocks) {
   const int64_t b = (n + 255) / 256;
   HK_REQUIRE(b < (1LL << 31), "too many elements (%lld)", (long long)n);
@@ -606,6 +624,57 @@ int hk_cast_linear_packed(const uint16_t* x, const uint16_t* w_packed, const flo
     ws.partial_elems = (workspace_bytes - kCastArrivals * 4) / 4;
   }
   return hk::gemm(g, ws, (hipStream_t)stream);
+}
+
+int hk_cast_linear_f32(const float* x, uint16_t* x_lp, const uint16_t* w, const uint16_t* bias,
+                       float* out, int M, int N, int K, int fmt, int packed, int min_work_groups,
+                       void* workspace, int64_t workspace_bytes, void* stream) {
+  constexpr int64_t kCastArrivals = 1 << 16;
+  HK_REQUIRE(x && x_lp && w && out, "hk_cast_linear_f32: null operand");
+  HK_REQUIRE(M >= 0 && N > 0 && K > 0 && K % 64 == 0,
+             "hk_cast_linear_f32: bad shape M=%d N=%d K=%d (K a multiple of 64)", M, N, K);
+  HK_REQUIRE(!packed || hk::packable(N, K),
+             "hk_cast_linear_f32: bad packed shape N=%d K=%d (N a multiple of 32, K of 64)", N, K);
+  HK_REQUIRE(fmt == hk::kLpBF16 || fmt == hk::kLpF16, "hk_cast_linear_f32: format %d", fmt);
+  HK_REQUIRE(hk::aligned16(x) && hk::aligned16(x_lp) && hk::aligned16(w),
+             "hk_cast_linear_f32: operands must be 16-byte aligned");
+  HK_REQUIRE(min_work_groups >= 0, "hk_cast_linear_f32: min_work_groups=%d", min_work_groups);
+  HK_REQUIRE(workspace == nullptr || workspace_bytes >= kCastArrivals * 4,
+             "hk_cast_linear_f32: a workspace needs at least %lld bytes",
+             (long long)kCastArrivals * 4);
+  if (M == 0) return HK_OK;
+  hipStream_t s = (hipStream_t)stream;
+  const int64_t n = (int64_t)M * K;
+  const unsigned blocks = (unsigned)std::min<int64_t>((n / 8 + 255) / 256, 2048);
+  if (fmt == hk::kLpF16)
+    hipLaunchKernelGGL(hk::cast_rows_kernel<hk::kLpF16>, dim3(blocks), dim3(256), 0, s, x, x_lp, n);
+  else
+    hipLaunchKernelGGL(hk::cast_rows_kernel<hk::kLpBF16>, dim3(blocks), dim3(256), 0, s, x, x_lp, n);
+  HK_LAUNCH_CHECK();
+  hk::GemmArgs g;
+  g.type = fmt == hk::kLpF16 ? hk::GemmType::kF16 : hk::GemmType::kBF16;
+  g.A = x_lp;
+  g.lda = K;
+  g.W = w;
+  g.ldw = K;
+  g.w_packed = packed != 0;
+  g.min_tiles = min_work_groups;
+  g.M = M;
+  g.N = N;
+  g.K = K;
+  g.ep.bias_lp = bias;
+  g.ep.round_lp = true;
+  g.ep.lp_fmt = fmt;
+  g.ep.out = out;
+  g.ep.ldo = N;
+  hk::GemmWorkspace ws;
+  if (workspace != nullptr) {
+    ws.arrivals = static_cast<int*>(workspace);
+    ws.arrival_elems = kCastArrivals;
+    ws.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCastArrivals * 4);
+    ws.partial_elems = (workspace_bytes - kCastArrivals * 4) / 4;
+  }
+  return hk::gemm(g, ws, s);
 }
 
 int hk_rglru_step(float* h, const float* x, const float* gate_i, const float* gate_r,

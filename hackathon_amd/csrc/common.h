@@ -156,10 +156,12 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ u32x4 gload16(const void* p) {
   return *(const __attribute__((address_space(1))) u32x4*)(p);
 }
+// (The whole vector is cast: __builtin_bit_cast of one element of a vector
+// reads element 0.)
 __device__ __forceinline__ float4 gload_f4(const float* p) {
-  const u32x4 v = gload16(p);
-  return make_float4(__builtin_bit_cast(float, v.x), __builtin_bit_cast(float, v.y),
-                     __builtin_bit_cast(float, v.z), __builtin_bit_cast(float, v.w));
+  typedef float f32x4v __attribute__((ext_vector_type(4)));
+  const f32x4v v = __builtin_bit_cast(f32x4v, gload16(p));
+  return make_float4(v.x, v.y, v.z, v.w);
 }
 __device__ __forceinline__ float gload(const float* p) {
   return *(const __attribute__((address_space(1))) float*)(p);

@@ -32,6 +32,7 @@ constexpr int kMinTilesShared = 112;
 
 struct GemmEpilogue {
   const float* bias = nullptr;      // [N] (per batch: + b*c_bstride)
+  const uint16_t* bias_lp = nullptr;  // or, 16-bit operands only: [N] in format lp_fmt
   const float* residual = nullptr;  // [M, ldr] added last
   int64_t ldr = 0;
   float* out = nullptr;             // fp32 result [M, ldo]

@@ -75,6 +75,14 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 constexpr int kBufWord3 = 0x00020000;
 constexpr int kCoherentSc1 = 16;
 
+// The bias of column n (fp32, or 16-bit widened exactly).
+__device__ __forceinline__ float bias_at(const GemmEpilogue& ep, int64_t n) {
+  if (ep.bias) return ep.bias[n];
+  if (ep.bias_lp)
+    return ep.lp_fmt == kLpF16 ? f16_bits_to_f32(ep.bias_lp[n]) : bf16_bits_to_f32(ep.bias_lp[n]);
+  return 0.0f;
+}
+
 // LDS address (byte offset) of a __shared__ object.
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
@@ -240,12 +248,10 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g, float* partial, i
   // The bias of this lane's two output columns, fetched before the slabs
   // (older than every transfer, so the counted waits cover it too).
   float bias_v[2] = {0.0f, 0.0f};
-  if (g.ep.bias) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = n0 + wn * 32 + j * 16 + fr;
-      if (n < g.N) bias_v[j] = g.ep.bias[n + (int)((int64_t)b * g.c_bstride)];
-    }
+  for (int j = 0; j < 2; ++j) {
+    const int n = n0 + wn * 32 + j * 16 + fr;
+    if (n < g.N) bias_v[j] = bias_at(g.ep, n + (int64_t)b * g.c_bstride);
   }
 
 #pragma unroll
@@ -787,7 +793,7 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void gemm_skinny_wp_kernel(GemmA
   // column exists)
   const int n = tn * 16 + fr;
   const GemmEpilogue& ep = g.ep;
-  const float bias_v = ep.bias ? ep.bias[n] : 0.0f;
+  const float bias_v = bias_at(ep, n);
   float v[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -921,9 +927,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_wp_kernel(GemmArgs g, float* par
   }
 
   float bias_v[2] = {0.0f, 0.0f};
-  if (g.ep.bias && cols_live) {
+  if (cols_live) {
 #pragma unroll
-    for (int c = 0; c < 2; ++c) bias_v[c] = g.ep.bias[nw0 + 16 * c + fr];
+    for (int c = 0; c < 2; ++c) bias_v[c] = bias_at(g.ep, nw0 + 16 * c + fr);
   }
 
   floatx4 acc[MF][2];

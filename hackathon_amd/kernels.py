@@ -269,17 +269,27 @@ def cast_linear(x, weight, bias=None, workspace=None, packed=False, min_work_gro
     dev = weight.device
     if dev.type != "cuda":
         raise _lib.HipLibraryError("cast_linear needs GPU tensors")
-    xl = x.reshape(-1, K).to(device=dev, dtype=weight.dtype).contiguous()
-    b = None
     if bias is not None:
         assert bias.dtype == weight.dtype and tuple(bias.shape) == (N,), "bias must be [N] in the weight's dtype"
-        b = bias.to(torch.float32).contiguous()
-    out = torch.empty(xl.shape[0], N, dtype=torch.float32, device=dev)
     ws, ws_bytes = None, 0
     if workspace is not None:
         assert workspace.dtype == torch.uint8 and workspace.device == dev
         ws, ws_bytes = workspace.data_ptr(), workspace.numel()
     lib = _lib.lib()
+    # fp32 rows on the weight's device: cast and product in one call
+    if (x.dtype == torch.float32 and x.device == dev and x.is_contiguous() and x.data_ptr() % 16 == 0
+            and (bias is None or (bias.device == dev and bias.is_contiguous()))):
+        M = x.numel() // max(K, 1)
+        xl = torch.empty(M, K, dtype=weight.dtype, device=dev)
+        out = torch.empty(M, N, dtype=torch.float32, device=dev)
+        _lib.check(lib.hk_cast_linear_f32(
+            x.data_ptr(), xl.data_ptr(), weight.data_ptr(), _lib.ptr(bias), out.data_ptr(), M, N, K,
+            _LP[weight.dtype], 1 if packed else 0, int(min_work_groups) if packed else 0, ws, ws_bytes,
+            _lib.current_stream(dev)), "hk_cast_linear_f32")
+        return out.reshape(*x.shape[:-1], N)
+    xl = x.reshape(-1, K).to(device=dev, dtype=weight.dtype).contiguous()
+    b = None if bias is None else bias.to(torch.float32).contiguous()
+    out = torch.empty(xl.shape[0], N, dtype=torch.float32, device=dev)
     if packed:
         st = lib.hk_cast_linear_packed(xl.data_ptr(), weight.data_ptr(), _lib.ptr(b), out.data_ptr(),
                                        xl.shape[0], N, K, _LP[weight.dtype], int(min_work_groups),

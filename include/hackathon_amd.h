@@ -119,6 +119,14 @@ int hk_cast_linear_packed(const uint16_t* x, const uint16_t* w_packed, const flo
                           float* out, int M, int N, int K, int fmt, int min_work_groups,
                           void* workspace, int64_t workspace_bytes, void* stream);
 
+/* CastLinear.forward with its casts (example_model.py:92-95): x [M, K] fp32 is
+ * rounded to format fmt into x_lp (scratch of M * K 16-bit values), multiplied
+ * by w (row-major, or with `packed` the hk_pack_cast_weight layout) and the
+ * 16-bit bias [N] (or null) added, as the two entries above. */
+int hk_cast_linear_f32(const float* x, uint16_t* x_lp, const uint16_t* w, const uint16_t* bias,
+                       float* out, int M, int N, int K, int fmt, int packed, int min_work_groups,
+                       void* workspace, int64_t workspace_bytes, void* stream);
+
 /* RGLRU.forward after its two BlockLinears (model/hawk.py:31-37):
  * i = sigmoid(gate_i), r = sigmoid(gate_r), a_t = a ** (c * r),
  * h <- h * a_t + sqrt(1 - a_t^2) * (i * x); out (NULL = none) = new h on
