@@ -934,6 +934,7 @@ int run_xlstm(Engine& e, TowerWS& w, int l, const Group& g, unsigned long long* 
   m.slot_ids = r.slot_ids;
   m.run_off = r.run_off;
   m.n_runs = r.n_runs;
+  m.n_long = r.n_long;
   m.alpha = {w.FG, d.nh, 1};
   m.scale = {w.IG, d.nh, 1};
   m.beta = {w.KS, I, d.hs_m};
@@ -977,6 +978,7 @@ int run_mamba2(Engine& e, int l, const Runs& r, hipStream_t s) {
   m.slot_ids = r.slot_ids;
   m.run_off = r.run_off;
   m.n_runs = r.n_runs;
+  m.n_long = r.n_long;
   m.alpha = {w.DEC, d.nhm, 1};
   m.scale = {w.DTS, d.nhm, 1};
   m.beta = {w.MXC + I, C, 0};
@@ -1015,6 +1017,7 @@ int run_retnet(Engine& e, int l, const Runs& r, hipStream_t s) {
   m.slot_ids = r.slot_ids;
   m.run_off = r.run_off;
   m.n_runs = r.n_runs;
+  m.n_long = r.n_long;
   m.alpha = {F32(e, kRetNet, l, R_DECAY), 0, 1};
   m.beta = {w.KR, H, d.hs_r};
   m.gamma = {w.QKVG + 2 * H, 4 * H, d.hs_r};
@@ -1263,6 +1266,7 @@ int xlstm_split_point(const int* run_off, int n_runs, double weight_us) {
 struct TickShape {
   int n_runs = 0, n_rows = 0, steps = 0;
   int split = 0, row_split = 0, steps2 = 0;
+  int n_long = 0;  // runs longer than the write-back log
   std::vector<int> act, act1, act2;
 };
 
@@ -1272,7 +1276,8 @@ struct TickShape {
 int enqueue_tick(Engine& e, const TickShape& sh, const float* features_dev, float* preds_dev,
                  hipStream_t s) {
   Group all;
-  all.r = Runs{e.d_slots, e.d_off, sh.n_runs, sh.n_rows, sh.steps, e.d_pos, e.d_rslot};
+  all.r = Runs{e.d_slots, e.d_off, sh.n_runs, sh.n_rows, sh.steps, e.d_pos, e.d_rslot,
+               sh.n_long};
   all.act_dev = e.d_act;
   all.act = sh.act;
   HK_TRY(stage_features(features_dev, sh.n_rows, e.d.F, e.d.Fpad, e.FE.f, e.FE.l, e.lp_fmt, s));
@@ -1281,11 +1286,13 @@ int enqueue_tick(Engine& e, const TickShape& sh, const float* features_dev, floa
   const bool split = sh.split < sh.n_runs;
   Group g1, g2;
   if (split) {
-    g1.r = Runs{e.d_slots, e.d_off, sh.split, sh.row_split, sh.steps, e.d_pos, e.d_rslot};
+    g1.r = Runs{e.d_slots, e.d_off, sh.split, sh.row_split, sh.steps, e.d_pos, e.d_rslot,
+                std::min(sh.n_long, sh.split)};
     g1.act_dev = e.d_act1;
     g1.act = sh.act1;
     g2.r = Runs{e.d_slots + sh.split, e.d_off2, sh.n_runs - sh.split, sh.n_rows - sh.row_split,
-                sh.steps2, e.d_pos + sh.row_split, e.d_rslot + sh.row_split};
+                sh.steps2, e.d_pos + sh.row_split, e.d_rslot + sh.row_split,
+                std::max(sh.n_long - sh.split, 0)};
     g2.act_dev = e.d_act2;
     g2.act = sh.act2;
     g2.row0 = sh.row_split;
@@ -1964,6 +1971,9 @@ int hk_engine_tick(void* h, const int* slot_ids_host, const int* run_off_host, i
   sh.split = split;
   sh.row_split = row_split;
   sh.steps2 = steps2;
+  while (sh.n_long < n_runs &&
+         run_off_host[sh.n_long + 1] - run_off_host[sh.n_long] > hk::kLogCapMax)
+    ++sh.n_long;
   sh.act.assign(h_act, h_act + steps);
   sh.act1.assign(h_act1, h_act1 + steps);
   sh.act2.assign(h_act2, h_act2 + steps2);

@@ -18,6 +18,7 @@ struct Runs {
   int max_len = 0;                // steps of the longest run (host)
   const int* row_pos = nullptr;   // device [n_rows]: position of each row in its run
   const int* row_slot = nullptr;  // device [n_rows]: slot of each row's run
+  int n_long = -1;                // runs longer than kLogCapMax steps (-1: not known)
 };
 
 // A width-4 causal conv (model/modules.py:23-49) computed by the kernel

@@ -63,6 +63,9 @@ struct MatScanDesc {
   float* log_b = nullptr;    // [slot][head][cap][rows]
   float* log_g = nullptr;    // [slot][head][cap][cols]
   int log_cap = 0;
+  // Runs with more than kLogCapMax steps: the first n_long (runs sorted by
+  // non-increasing length); -1 when the caller does not know them.
+  int n_long = -1;
 };
 
 // The log-header update of one scan launch (deferred write-back), as a job
@@ -127,6 +130,11 @@ __device__ __forceinline__ void log_commit_one(const LogCommit& c, int i) {
 LogCommit log_commit_of(const MatScanDesc& d);
 
 int launch_mat_scan(const MatScanDesc& d, hipStream_t stream);
+// The streaming scan (scan_stream.hip) and the launches it takes: its runs
+// have at most kLogCapMax steps (launch_mat_scan hands the first n_long to the
+// general kernel).
+bool stream_scan_takes(const MatScanDesc& d);
+int launch_stream_scan(const MatScanDesc& d, hipStream_t stream);
 // The LogCommit job of a scan launch as a launch of its own; run after it.
 int launch_mat_log_commit(const MatScanDesc& d, hipStream_t stream);
 // Materialises slots [slot0, slot0 + n) into B and empties their logs.

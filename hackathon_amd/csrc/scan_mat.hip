@@ -589,6 +589,20 @@ int launch_mat_scan(const MatScanDesc& d, hipStream_t stream) {
              "mat_scan: tile too large for 32-bit byte offsets");
   if (d.n_runs == 0) return HK_OK;
   HK_REQUIRE(d.n_runs <= 65535, "mat_scan: at most 65535 runs per launch");
+  if (stream_scan_takes(d)) {
+    if (d.n_long > 0) {
+      MatScanDesc l = d;
+      l.n_runs = d.n_long;
+      l.n_long = -1;
+      const int st = launch_mat_scan(l, stream);
+      if (st != HK_OK) return st;
+    }
+    MatScanDesc q = d;
+    q.slot_ids += d.n_long;
+    q.run_off += d.n_long;
+    q.n_runs -= d.n_long;
+    return launch_stream_scan(q, stream);
+  }
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   const bool vec = prows % 4 == 0 && al16(d.beta.ptr) && al16(d.w.ptr) &&
                    d.beta.row_stride % 4 == 0 && d.beta.head_stride % 4 == 0 &&
