@@ -536,7 +536,8 @@ def xlstm_split_point(run_off, weight_us=0.0):
     longest run plus 5 us per symbol, a split charged one more read of a
     layer's weights (weight_us), split when the larger group's cost plus
     that read is under 0.8 of the whole), for ticks whose longest run has at
-    least 16 requests; the engine keeps shorter ones whole. Returns the first run of the
+    least 16 requests, as the replayed ticks have; the engine keeps ticks of
+    shorter runs whole below 192 runs. Returns the first run of the
     second group (len(runs) for no split)."""
     n = len(run_off) - 1
     if n < 2:

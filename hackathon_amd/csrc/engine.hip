@@ -1235,16 +1235,20 @@ int run_towers_mt(Engine& e, const Group& all, const Group& g1, const Group* g2,
 // bf16 (C4): about 1000 against 500 + 24.)
 // The second group also takes the stream that Hawk would have, so it has to
 // shorten a long chain of sLSTM steps: ticks whose longest run is below
-// kSplitMinLen stay whole. Two-layer ticks, us split / whole: 32, 64 and 256
+// kSplitMinLen stay whole (until they have very many runs, below). Two-layer ticks, us split / whole: 32, 64 and 256
 // single requests 685 / 637, 888 / 873 and 2349 / 2285; 256 with runs of up
 // to about six 2011 / 1968; 64 single requests in fp32 1309 / 1167; with a
-// run of about fifty 256 requests 1500 / 1574 and 800 3347 / 3629.
+// run of about fifty 256 requests 1500 / 1574 and 800 3347 / 3629. From
+// kSplitMinRuns runs up two groups pay again: one group's scan reads HBM while
+// the other's projections keep the matrix cores busy (whole / split, back to back: 256
+// runs 2220 / 2147 us, 512 4130 / 3990, 610 5690 / 5365; 128 runs 1358 / 1492).
 constexpr int kSplitMinLen = 16;
+constexpr int kSplitMinRuns = 192;
 int xlstm_split_point(const int* run_off, int n_runs, double weight_us) {
   constexpr double kStepUs = 3.0, kSymbolUs = 5.0, kGain = 0.8;
   if (n_runs < 2) return n_runs;
   const int len0 = run_off[1] - run_off[0];
-  if (len0 < kSplitMinLen) return n_runs;
+  if (len0 < kSplitMinLen && n_runs < kSplitMinRuns) return n_runs;
   const double whole = kStepUs * len0 + kSymbolUs * n_runs;
   double best = whole;
   int best_k = n_runs;
