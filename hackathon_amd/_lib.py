@@ -105,6 +105,11 @@ def ptr(t) -> int:
 
 
 def current_stream(device) -> int:
+    """The raw handle of torch's current stream on a CUDA device. Taken from
+    the binding torch.cuda.current_stream wraps: every operator call asks for
+    it, and the Stream object costs the call about as much as its checks."""
     import torch
 
-    return torch.cuda.current_stream(device).cuda_stream
+    if device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
