@@ -12,7 +12,8 @@
 // fp32 products of at most 16 rows (any batch description, every epilogue;
 // split_wscale is not used there: exact fp32), and packed 16-bit
 // projections of at most 16 rows, run on kernels of their own that stream W
-// through registers without splitting K.
+// through registers without splitting K. Exact fp32 products of more rows with
+// a short K and few 64x64 tiles run on a kernel of smaller tiles.
 #pragma once
 
 #include "common.h"
