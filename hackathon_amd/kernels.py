@@ -277,8 +277,10 @@ def cast_linear(x, weight, bias=None, workspace=None, packed=False, min_work_gro
         ws, ws_bytes = workspace.data_ptr(), workspace.numel()
     lib = _lib.lib()
     # fp32 rows on the weight's device: cast and product in one call
+    # (not a lazily negated view: its memory holds the other sign)
     if (x.dtype == torch.float32 and x.device == dev and x.is_contiguous() and x.data_ptr() % 16 == 0
-            and (bias is None or (bias.device == dev and bias.is_contiguous()))):
+            and not x.is_neg()
+            and (bias is None or (bias.device == dev and bias.is_contiguous() and not bias.is_neg()))):
         M = x.numel() // max(K, 1)
         xl = torch.empty(M, K, dtype=weight.dtype, device=dev)
         out = torch.empty(M, N, dtype=torch.float32, device=dev)

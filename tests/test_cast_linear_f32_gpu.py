@@ -2,7 +2,7 @@
 bits of the separate casts for every layout: odd row counts, both weight
 layouts, with and without bias, values outside the 16-bit range, infinities
 and NaN, rows that are a view at an unaligned address (which take the separate
-casts) and rows in another type."""
+casts), rows in another type and lazily negated views."""
 
 import pytest
 import torch
@@ -34,3 +34,6 @@ def test_one_call_equals_separate_casts(dev, dtype, M, N, K):
             want = hk.cast_linear(x, weight, bias, packed=p)
             assert torch.equal(hk.cast_linear(shifted, weight, bias, packed=p), want)
             assert torch.equal(hk.cast_linear(x.view(1, M, K), weight, bias, packed=p)[0], want)
+    want = hk.cast_linear(-x, w, -b)
+    assert torch.equal(hk.cast_linear(torch._neg_view(x), w, -b), want)
+    assert torch.equal(hk.cast_linear(-x, w, torch._neg_view(b)), want)
