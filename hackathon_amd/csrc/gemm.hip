@@ -77,10 +77,12 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 constexpr int kBufWord3 = 0x00020000;
 constexpr int kCoherentSc1 = 16;
 
-// The bias of column n (fp32, or 16-bit widened exactly).
+// The bias of column n (fp32, or with LP 16-bit widened exactly; fp32 products
+// leave that form out).
+template <bool LP = true>
 __device__ __forceinline__ float bias_at(const GemmEpilogue& ep, int64_t n) {
   if (ep.bias) return ep.bias[n];
-  if (ep.bias_lp)
+  if (LP && ep.bias_lp)
     return ep.lp_fmt == kLpF16 ? f16_bits_to_f32(ep.bias_lp[n]) : bf16_bits_to_f32(ep.bias_lp[n]);
   return 0.0f;
 }
@@ -250,10 +252,13 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g, float* partial, i
   // The bias of this lane's two output columns, fetched before the slabs
   // (older than every transfer, so the counted waits cover it too).
   float bias_v[2] = {0.0f, 0.0f};
+  if (g.ep.bias || (T != GemmType::kF32 && g.ep.bias_lp)) {
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int n = n0 + wn * 32 + j * 16 + fr;
-    if (n < g.N) bias_v[j] = bias_at(g.ep, n + (int64_t)b * g.c_bstride);
+    for (int j = 0; j < 2; ++j) {
+      const int n = n0 + wn * 32 + j * 16 + fr;
+      if (n < g.N)
+        bias_v[j] = bias_at<T != GemmType::kF32>(g.ep, n + (int)((int64_t)b * g.c_bstride));
+    }
   }
 
 #pragma unroll
