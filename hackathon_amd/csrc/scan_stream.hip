@@ -8,7 +8,8 @@
 // steps are one list of at most 16 rank-1 entries (b_j, g_j), and
 //   out_t = P_t F (w_t . B) + sum_j c_tj (w_t . b_j) g_j,
 // with P_t the product of the alphas up to t and c_tj = P_t a_j for a log
-// entry, the product of the alphas after s for step s <= t (0 past t). So a
+// entry, the product of the alphas after s for step s <= t (the sum ends
+// there: a step's output never reads a later step's operands). So a
 // run that leaves its tile in the store (its steps fit the log) reads the
 // tile once and spends one multiply-add per element and step: nothing is
 // applied to the tile and nothing of it is kept, where mat_scan_kernel applies
@@ -236,8 +237,10 @@ struct Tile {
 #pragma unroll 1
       for (int v = 0; v < waves; ++v) s += lb[v * kEnt * 64 + q * CT + c];
       float o = lcd[t * (kEnt + 1) + kEnt] * s;
+      // up to the step's own entry: a later one's weight is zero, but zero times
+      // an infinity or NaN that came with a later request is not
 #pragma unroll 1
-      for (int j = 0; j < k.ne; ++j) o = fmaf(lcd[t * (kEnt + 1) + j], lg[j * CT + c], o);
+      for (int j = 0; j <= k.n + t; ++j) o = fmaf(lcd[t * (kEnt + 1) + j], lg[j * CT + c], o);
       gstore(ob + (k.row0 + t) * d.out_row_stride, o);
     }
   }

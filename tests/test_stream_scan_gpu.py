@@ -63,3 +63,37 @@ def test_ticks_match_reference_rounds(dev, params, lens):
     g, w32, w64 = cat(got), cat(p32), cat(p64)
     err, ref = (np.linalg.norm(v - w64, axis=0) for v in (g, w32))
     assert (err <= 2.0 * ref).all(), (err, ref)
+
+
+@pytest.mark.parametrize("dtype,bad", [("fp32", np.inf), ("bf16", -np.inf), ("fp16", 1e5)])
+def test_a_bad_request_leaves_the_earlier_answers(dev, params, dtype, bad):
+    """A request with a feature that is infinite, or beyond fp16's range,
+    spoils its own answer and no other: the earlier requests of its run, in
+    the same tick, and every other symbol are answered bit for bit as without
+    it, with logs empty, partly filled and full (so that tiles stay and are
+    written back)."""
+    from hackathon_amd.engine import Engine, Runs
+
+    lens = sorted(SHORT + [1] * (64 - len(SHORT)), reverse=True)
+    n, rows = len(lens), sum(lens)
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    last = off[1:] - 1
+    eng = Engine(CFG, capacity=2 * n, max_rows=rows, linear_dtype=dtype)
+    eng.load_weights(params)
+    rng = np.random.default_rng(1)
+    x = lambda: np.clip(rng.standard_normal((rows, CFG.num_features)), -5, 5).astype(np.float32)
+    tick = lambda slot0, f: eng.tick(Runs(np.arange(slot0, slot0 + n, dtype=np.int32), off),
+                                     torch.from_numpy(f).to(dev)).cpu().numpy()
+    for fill in range(3):
+        eng.copy_slots(0, n, n)
+        good = x()
+        spoilt = good.copy()
+        spoilt[last[:16], 0] = bad  # the runs of two steps and more
+        want, got = tick(0, good), tick(n, spoilt)
+        assert not np.isfinite(got[last[:16]]).all()
+        keep = np.ones(rows, bool)
+        keep[last[:16]] = False
+        assert np.isfinite(want).all()
+        assert np.array_equal(got[keep], want[keep]), fill
+    eng.check()
+    eng.close()
