@@ -662,7 +662,8 @@ int hk_cast_linear_f32(const float* x, uint16_t* x_lp, const uint16_t* w, const 
   g.M = M;
   g.N = N;
   g.K = K;
-  g.ep.bias_lp = bias;
+  g.ep.bias = reinterpret_cast<const float*>(bias);
+  g.ep.bias_lp = bias != nullptr;
   g.ep.round_lp = true;
   g.ep.lp_fmt = fmt;
   g.ep.out = out;

@@ -33,7 +33,6 @@ constexpr int kMinTilesShared = 112;
 
 struct GemmEpilogue {
   const float* bias = nullptr;      // [N] (per batch: + b*c_bstride)
-  const uint16_t* bias_lp = nullptr;  // or, 16-bit operands only: [N] in format lp_fmt
   const float* residual = nullptr;  // [M, ldr] added last
   int64_t ldr = 0;
   float* out = nullptr;             // fp32 result [M, ldo]
@@ -42,6 +41,7 @@ struct GemmEpilogue {
   int64_t ldl = 0;
   int lp_fmt = kLpBF16;             // LpFmt of round_lp and out_lp
   bool round_lp = false;            // round (acc + bias) to lp_fmt first
+  bool bias_lp = false;             // 16-bit operands only: bias points at [N] values in lp_fmt
   int act = 0;                      // 0 none, 1 relu (after rounding)
   // Mamba2's dt (model/mamba2.py:92-97), fp32 products only: with dt_a set
   // the result is dt = softplus(acc + bias) (in out), and

@@ -77,14 +77,10 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 constexpr int kBufWord3 = 0x00020000;
 constexpr int kCoherentSc1 = 16;
 
-// The bias of column n (fp32, or with LP 16-bit widened exactly; fp32 products
-// leave that form out).
-template <bool LP = true>
-__device__ __forceinline__ float bias_at(const GemmEpilogue& ep, int64_t n) {
-  if (ep.bias) return ep.bias[n];
-  if (LP && ep.bias_lp)
-    return ep.lp_fmt == kLpF16 ? f16_bits_to_f32(ep.bias_lp[n]) : bf16_bits_to_f32(ep.bias_lp[n]);
-  return 0.0f;
+// A 16-bit bias (GemmEpilogue::bias_lp), widened exactly.
+__device__ __forceinline__ float bias_lp_at(const GemmEpilogue& ep, int64_t n) {
+  const uint16_t v = reinterpret_cast<const uint16_t*>(ep.bias)[n];
+  return ep.lp_fmt == kLpF16 ? f16_bits_to_f32(v) : bf16_bits_to_f32(v);
 }
 
 // LDS address (byte offset) of a __shared__ object.
@@ -252,12 +248,17 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g, float* partial, i
   // The bias of this lane's two output columns, fetched before the slabs
   // (older than every transfer, so the counted waits cover it too).
   float bias_v[2] = {0.0f, 0.0f};
-  if (g.ep.bias || (T != GemmType::kF32 && g.ep.bias_lp)) {
+  if (T != GemmType::kF32 && g.ep.bias_lp) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int n = n0 + wn * 32 + j * 16 + fr;
-      if (n < g.N)
-        bias_v[j] = bias_at<T != GemmType::kF32>(g.ep, n + (int)((int64_t)b * g.c_bstride));
+      if (n < g.N) bias_v[j] = bias_lp_at(g.ep, n + (int)((int64_t)b * g.c_bstride));
+    }
+  } else if (g.ep.bias) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int n = n0 + wn * 32 + j * 16 + fr;
+      if (n < g.N) bias_v[j] = g.ep.bias[n + (int)((int64_t)b * g.c_bstride)];
     }
   }
 
@@ -800,7 +801,7 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void gemm_skinny_wp_kernel(GemmA
   // column exists)
   const int n = tn * 16 + fr;
   const GemmEpilogue& ep = g.ep;
-  const float bias_v = bias_at(ep, n);
+  const float bias_v = ep.bias_lp ? bias_lp_at(ep, n) : ep.bias ? ep.bias[n] : 0.0f;
   float v[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -933,10 +934,17 @@ __global__ __launch_bounds__(64 * NW) void gemm_wp_kernel(GemmArgs g, float* par
     akey[i] = (ra >> 1) & 7;
   }
 
+  // A uniform branch for each form of the bias, so that a launch with the
+  // fp32 bias or none waits for nothing here (one helper for both inside the
+  // column loop cost every launch of the kernel 0.2-0.4 us: 256x8192x2048
+  // 17.73, with the branches 17.40).
   float bias_v[2] = {0.0f, 0.0f};
-  if (cols_live) {
+  if (cols_live && g.ep.bias_lp) {
 #pragma unroll
-    for (int c = 0; c < 2; ++c) bias_v[c] = bias_at(g.ep, nw0 + 16 * c + fr);
+    for (int c = 0; c < 2; ++c) bias_v[c] = bias_lp_at(g.ep, nw0 + 16 * c + fr);
+  } else if (cols_live && g.ep.bias) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) bias_v[c] = g.ep.bias[nw0 + 16 * c + fr];
   }
 
   floatx4 acc[MF][2];
@@ -1422,6 +1430,8 @@ int gemm(const GemmArgs& g, const GemmWorkspace& ws, hipStream_t stream, int spl
   HK_REQUIRE(g.split_wscale == 0.0f ||
                  (std::isfinite(g.split_wscale) && std::frexp(g.split_wscale, &wexp) == 0.5f),
              "gemm: split_wscale %g is not a positive power of two", (double)g.split_wscale);
+  HK_REQUIRE(!g.ep.bias_lp || (g.ep.bias && g.type != GemmType::kF32),
+             "gemm: a 16-bit bias needs 16-bit operands");
   const bool narrow = g.type == GemmType::kF32 && g.K % Tr<GemmType::kF32>::BK != 0;
   const bool half = g.type != GemmType::kF32;  // bf16 or fp16 operands
   const int BK = half     ? Tr<GemmType::kBF16>::BK
