@@ -527,6 +527,7 @@ int hk_block_linear(const float* x, const float* weight, const float* bias, floa
     g.a_bstride = block_size;
     g.w_bstride = (int64_t)block_size * block_size;
     g.c_bstride = block_size;
+    g.alone = true;
     g.ep.bias = bias;
     g.ep.out = out;
     g.ep.ldo = (int64_t)blocks * block_size;

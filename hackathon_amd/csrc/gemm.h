@@ -13,7 +13,8 @@
 // split_wscale is not used there: exact fp32), and packed 16-bit
 // projections of at most 16 rows, run on kernels of their own that stream W
 // through registers without splitting K. Exact fp32 products of more rows with
-// a short K and few 64x64 tiles run on a kernel of smaller tiles.
+// a short K and few 64x64 tiles run on a kernel of smaller tiles where the
+// caller says that they have the device to themselves (GemmArgs::alone).
 #pragma once
 
 #include "common.h"
@@ -71,6 +72,9 @@ struct GemmArgs {
   // 16-bit W held in the fragment-packed layout of pack_lp_weight (ldw is
   // then unused; N and K must be multiples of 32 and 64).
   bool w_packed = false;
+  // fp32 operands: no other stream shares the device (an operator call; a
+  // tick's products run beside three other streams and leave it unset).
+  bool alone = false;
   // Packed kernel's tile rule: the largest tile that still gives at least
   // this many work-groups without splitting K (0: kMinTilesAlone, for a GEMM
   // that has the device to itself; the engine's ticks, where three other

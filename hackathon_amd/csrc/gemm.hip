@@ -6,8 +6,8 @@
 //   BlockLinear batches) and 16-bit weights in row-major layout;
 // - gemm_skinny_kernel and gemm_skinny_wp_kernel, for fp32 products and
 //   packed 16-bit projections of at most 16 rows (described at the kernels);
-// - gemm_block_kernel, for exact fp32 products of more rows whose K is short
-//   and whose 64x64 tiles are few (described at the kernel).
+// - gemm_block_kernel, for an operator call's exact fp32 products of more rows
+//   whose K is short and whose 64x64 tiles are few (described at the kernel).
 //
 // gemm_kernel: 64x64 output tile per 256-thread work-group, 4 wave64s in a 2x2 layout,
 // each wave owning a 32x32 sub-tile = 2x2 MFMA 16x16 fragments. K advances in
@@ -628,20 +628,24 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void gemm_skinny_kernel(GemmArgs
   store_f32_fragment(g, b, 4 * fk, n0 + fr, acc);
 }
 
-// BlockLinear products of more than 16 rows (fp32, K at most kBlockK): a
+// BlockLinear operator calls of more than 16 rows (fp32, K at most kBlockK): a
 // launch has few 64x64 tiles (64 rows of four 512-wide blocks: 32) and K is
 // too short to split over work-groups, so gemm_kernel left most CUs idle and
-// ran each tile's K as one chain of slabs (64 rows 14.6 us, 256 rows 15.8).
+// ran each tile's K as one chain of slabs (64 rows 14.5 us, 256 rows 14.6).
 // Here a work-group of 8 waves owns a 16 MT x 16 NT tile and all of K; the
 // waves take interleaved 16-deep k steps, kBlockU of them loaded together
 // straight into registers (A and W fragments, 16 rows x 64 bytes each), and
 // their sums meet in LDS, added in wave order, one fragment per wave. What
 // bounds it: one load latency, the products and the sum in LDS, one after the
 // other in each work-group. Measured (512-wide blocks, four of them, us, this
-// kernel / gemm_kernel): 32 rows 5.1 / 14.3, 64 6.3 / 14.4, 128 9.0 / 14.6, 256
-// 11.4 / 15.0; against float64 its error is 0.4 of gemm_kernel's (shorter
+// kernel / gemm_kernel): 32 rows 5.4 / 14.3, 64 6.4 / 14.5, 128 8.6 / 14.5, 256
+// 10.8 / 14.6; against float64 its error is 0.4 of gemm_kernel's (shorter
 // chains of sums). At kBlockTiles 64x64 tiles and more gemm_kernel fills the
-// device and is faster (384 rows 15.4 / 20.6, 1000 rows 26.5 / 39.8).
+// device (see also block_tile). Inside a tick, whose other streams hold most
+// CUs, gemm_kernel's few work-groups cost less: fp32 ticks with this kernel /
+// without, two layers, 32 requests of 32 symbols 923 / 905 us, 64 of 64 1153 /
+// 1136, 81 of 48 1554 / 1533; twelve layers 4911 / 4885, 6358 / 6326, 8386 /
+// 8317.
 constexpr int kBlockWaves = 8;
 constexpr int kBlockU = 4;
 constexpr int kBlockK = 512;
@@ -1358,31 +1362,51 @@ int gemm_skinny(const GemmArgs& g, hipStream_t stream) {
   return HK_OK;
 }
 
-// fp32 products of more than kSkinnyRows rows with a short K (any batch
-// description).
-int gemm_block(const GemmArgs& g, hipStream_t stream) {
-  // The largest of 64x32, 64x16, 32x16 and 16x16 (rows x columns) that still
-  // gives 192 work-groups, most of the 256 CUs (asking for 320 takes smaller
-  // tiles, which read more: 256 rows 14.3 against 11.4 us).
-  static const int kTiles[4][2] = {{4, 2}, {4, 1}, {2, 1}, {1, 1}};  // (MT, NT)
-  auto tiles = [&](int c) {
-    return (int64_t)((g.M + 16 * kTiles[c][0] - 1) / (16 * kTiles[c][0])) *
-           ((g.N + 16 * kTiles[c][1] - 1) / (16 * kTiles[c][1])) * g.batch;
+// Tile of gemm_block_kernel for the product (MT x NT fragments), or false
+// where gemm_kernel is the faster one. The largest of 64x32, 64x16, 32x16 and
+// 16x16 (rows x columns) that still gives 192 work-groups, most of the 256 CUs
+// (asking for 320 takes smaller tiles, which read more: 256 rows 14.3 against
+// 11.4 us). A CU holds one work-group of the 64-row tiles (registers), so
+// those have to come to at most kBlockCUs: a second turn doubles the launch
+// (four 512-wide blocks, this kernel / gemm_kernel: 256 rows, 256 work-groups
+// 10.8 / 14.6 us, 257 rows, 320 work-groups 19.2 / 14.7; 256-wide, one block:
+// 2048 rows 9.1 / 9.7, 2176 rows 16.3 / 9.7). Then the 64x16 tile gives way to
+// 64x32, which halves its work-groups, and 64x32 to gemm_kernel. The smaller
+// tiles share CUs and stay ahead up to their 383 work-groups (128-wide: 1.0 to
+// 0.7 of gemm_kernel's time, 512-wide 0.6 to 0.4).
+constexpr int kBlockCUs = 256;
+struct BlockTile {
+  int mt, nt;
+};
+bool block_tile(int M, int N, int batch, BlockTile* out) {
+  static const BlockTile kTiles[4] = {{4, 2}, {4, 1}, {2, 1}, {1, 1}};
+  auto groups = [&](int c) {
+    return (int64_t)((M + 16 * kTiles[c].mt - 1) / (16 * kTiles[c].mt)) *
+           ((N + 16 * kTiles[c].nt - 1) / (16 * kTiles[c].nt)) * batch;
   };
   int pick = 0;
-  while (pick < 3 && tiles(pick) < 192) ++pick;
-  HK_REQUIRE(tiles(pick) < (1LL << 31), "gemm: grid too large");
-  const int mt = kTiles[pick][0], nt = kTiles[pick][1];
-  const int tiles_m = (g.M + 16 * mt - 1) / (16 * mt);
-  const int tiles_n = (g.N + 16 * nt - 1) / (16 * nt);
-  const dim3 grid((unsigned)tiles(pick)), block(64 * kBlockWaves);
+  while (pick < 3 && groups(pick) < 192) ++pick;
+  if (pick == 1 && groups(pick) > kBlockCUs) pick = 0;
+  if (pick == 0 && groups(pick) > kBlockCUs) return false;
+  *out = kTiles[pick];
+  return true;
+}
+
+// fp32 products of more than kSkinnyRows rows with a short K (any batch
+// description).
+int gemm_block(const GemmArgs& g, const BlockTile& t, hipStream_t stream) {
+  const int tiles_m = (g.M + 16 * t.mt - 1) / (16 * t.mt);
+  const int tiles_n = (g.N + 16 * t.nt - 1) / (16 * t.nt);
+  const int64_t nwg = (int64_t)tiles_m * tiles_n * g.batch;
+  HK_REQUIRE(nwg < (1LL << 31), "gemm: grid too large");
+  const dim3 grid((unsigned)nwg), block(64 * kBlockWaves);
 #define HK_BLOCK(MT, NT)                                                                         \
   hipLaunchKernelGGL((gemm_block_kernel<MT, NT>), grid, block, 0, stream, g, tiles_m, tiles_n)
-  if (pick == 0) {
+  if (t.mt == 4 && t.nt == 2) {
     HK_BLOCK(4, 2);
-  } else if (pick == 1) {
+  } else if (t.mt == 4) {
     HK_BLOCK(4, 1);
-  } else if (pick == 2) {
+  } else if (t.mt == 2) {
     HK_BLOCK(2, 1);
   } else {
     HK_BLOCK(1, 1);
@@ -1449,8 +1473,10 @@ int gemm(const GemmArgs& g, const GemmWorkspace& ws, hipStream_t stream, int spl
   const int tiles_n = (g.N + BN - 1) / BN;
   const int64_t tiles = (int64_t)tiles_m * tiles_n * g.batch;
   // A short K and too few 64x64 tiles to fill the device (kBlockTiles).
-  if (g.type == GemmType::kF32 && g.split_wscale == 0.0f && g.K <= kBlockK && tiles < kBlockTiles)
-    return gemm_block(g, stream);
+  BlockTile block;
+  if (g.type == GemmType::kF32 && g.alone && g.split_wscale == 0.0f && g.K <= kBlockK &&
+      tiles < kBlockTiles && block_tile(g.M, g.N, g.batch, &block))
+    return gemm_block(g, block, stream);
   const int ktiles = g.K / BK;
   int splits = splits_hint;
   if (splits <= 0) {
