@@ -823,6 +823,19 @@ int row_parts(const Runs& r, int rows) {
   return p;
 }
 
+// The scan of tower t's matrix state at layer l over runs r, without its
+// operands. (Mamba2's rows are not split: its 128-row tile leaves too little
+// work per part, and its stream is not the one that ends the tick.)
+MatScanDesc run_scan_desc(const Engine& e, int t, int l, const Runs& r) {
+  MatScanDesc m = mat_state_desc(e, t, l);
+  m.slot_ids = r.slot_ids;
+  m.run_off = r.run_off;
+  m.n_runs = r.n_runs;
+  m.n_long = r.n_long;
+  m.row_parts = t == kMamba2 ? 1 : row_parts(r, m.rows);
+  return m;
+}
+
 int timed_mat_scan(Engine& e, int kind, const MatScanDesc& m, hipStream_t s) {
   return timed(e, kind, s, [&] { return launch_mat_scan(m, s); });
 }
@@ -930,11 +943,7 @@ int run_xlstm(Engine& e, TowerWS& w, int l, const Group& g, unsigned long long* 
     HK_TRY(mlstm_gates(r, w.IF, 1, 0, d.nh, w.QKV, I, w.KS, st[XS_L_N], st[XS_L_M], w.IG, w.FG,
                        w.DEN, s));
   }
-  MatScanDesc m = mat_state_desc(e, kXLSTM, l);
-  m.slot_ids = r.slot_ids;
-  m.run_off = r.run_off;
-  m.n_runs = r.n_runs;
-  m.n_long = r.n_long;
+  MatScanDesc m = run_scan_desc(e, kXLSTM, l, r);
   m.alpha = {w.FG, d.nh, 1};
   m.scale = {w.IG, d.nh, 1};
   m.beta = {w.KS, I, d.hs_m};
@@ -943,7 +952,6 @@ int run_xlstm(Engine& e, TowerWS& w, int l, const Group& g, unsigned long long* 
   m.out = w.NUM;
   m.out_row_stride = I;
   m.out_head_stride = d.hs_m;
-  m.row_parts = row_parts(r, d.hs_m);
   m.out_part_stride = (int64_t)n * I;
   HK_TRY(timed_mat_scan(e, 0, m, s));
   HK_TRY(mlstm_post(w.NUM, m.row_parts, m.out_part_stride, w.DEN, d.nh, F32(e, kXLSTM, l, X_L_GN_W), F32(e, kXLSTM, l, X_L_GN_B),
@@ -974,11 +982,7 @@ int run_mamba2(Engine& e, int l, const Runs& r, hipStream_t s) {
                 F32(e, kMamba2, l, M_A), w.DEC));
   HK_TRY(conv_scan(r, w.PROJ, W, C, st[MS_CONV], le[MS_CONV], F32(e, kMamba2, l, M_CONV_W),
                    F32(e, kMamba2, l, M_CONV_B), 1, w.MXC, C, s));
-  MatScanDesc m = mat_state_desc(e, kMamba2, l);
-  m.slot_ids = r.slot_ids;
-  m.run_off = r.run_off;
-  m.n_runs = r.n_runs;
-  m.n_long = r.n_long;
+  MatScanDesc m = run_scan_desc(e, kMamba2, l, r);
   m.alpha = {w.DEC, d.nhm, 1};
   m.scale = {w.DTS, d.nhm, 1};
   m.beta = {w.MXC + I, C, 0};
@@ -987,8 +991,6 @@ int run_mamba2(Engine& e, int l, const Runs& r, hipStream_t s) {
   m.out = w.YS;
   m.out_row_stride = I;
   m.out_head_stride = d.hm;
-  // (not split: the 128-row tile leaves too little work per part, and this
-  // tower's stream is not the one that ends the tick)
   m.out_part_stride = (int64_t)n * I;
   HK_TRY(timed_mat_scan(e, 1, m, s));
   HK_TRY(mamba2_post(w.YS, m.row_parts, m.out_part_stride, w.MXC, C, w.PROJ + C, W, F32(e, kMamba2, l, M_D),
@@ -1013,11 +1015,7 @@ int run_retnet(Engine& e, int l, const Runs& r, hipStream_t s) {
   HK_TRY(retnet_prep(r, w.QKVG, 4 * H, H, d.nh, scaling, F32(e, kRetNet, l, R_ANGLE),
                      F32(e, kRetNet, l, R_DECAY), reinterpret_cast<int*>(st[RS_OFF]),
                      st[RS_SCALE], w.KR, w.QS, s));
-  MatScanDesc m = mat_state_desc(e, kRetNet, l);
-  m.slot_ids = r.slot_ids;
-  m.run_off = r.run_off;
-  m.n_runs = r.n_runs;
-  m.n_long = r.n_long;
+  MatScanDesc m = run_scan_desc(e, kRetNet, l, r);
   m.alpha = {F32(e, kRetNet, l, R_DECAY), 0, 1};
   m.beta = {w.KR, H, d.hs_r};
   m.gamma = {w.QKVG + 2 * H, 4 * H, d.hs_r};
@@ -1025,7 +1023,6 @@ int run_retnet(Engine& e, int l, const Runs& r, hipStream_t s) {
   m.out = w.O;
   m.out_row_stride = H;
   m.out_head_stride = d.hs_r;
-  m.row_parts = row_parts(r, d.hs_r);
   m.out_part_stride = (int64_t)n * H;
   HK_TRY(timed_mat_scan(e, 2, m, s));
   // the slots' offsets and scales advance after every reader (retnet_prep)
@@ -1274,14 +1271,42 @@ struct TickShape {
   std::vector<int> act, act1, act2;
 };
 
+// The layout part of a tick's shape, from its length-sorted runs.
+TickShape tick_shape(const Engine& e, const int* run_off, int n_runs) {
+  TickShape sh;
+  sh.n_runs = n_runs;
+  sh.n_rows = run_off[n_runs];
+  sh.steps = run_off[1] - run_off[0];
+  // xLSTM run groups: runs [0, split) and [split, n_runs).
+  sh.split = xlstm_split_point(run_off, n_runs, e.x_weight_us);
+  sh.row_split = run_off[sh.split];
+  sh.steps2 = sh.split < n_runs ? run_off[sh.split + 1] - run_off[sh.split] : 0;
+  while (sh.n_long < n_runs && run_off[sh.n_long + 1] - run_off[sh.n_long] > kLogCapMax)
+    ++sh.n_long;
+  return sh;
+}
+
+// The runs of the whole tick, and of its xLSTM groups when it is split.
+Runs all_runs(const Engine& e, const TickShape& sh) {
+  return Runs{e.d_slots, e.d_off, sh.n_runs, sh.n_rows, sh.steps, e.d_pos, e.d_rslot, sh.n_long};
+}
+Runs group1_runs(const Engine& e, const TickShape& sh) {
+  return Runs{e.d_slots, e.d_off, sh.split, sh.row_split, sh.steps, e.d_pos, e.d_rslot,
+              std::min(sh.n_long, sh.split)};
+}
+Runs group2_runs(const Engine& e, const TickShape& sh) {
+  return Runs{e.d_slots + sh.split, e.d_off2, sh.n_runs - sh.split, sh.n_rows - sh.row_split,
+              sh.steps2, e.d_pos + sh.row_split, e.d_rslot + sh.row_split,
+              std::max(sh.n_long - sh.split, 0)};
+}
+
 // The device work of one tick on stream s, descriptors already in d_desc:
 // feature staging, every tower (forked to the side streams and joined back),
 // predictions into preds_dev.
 int enqueue_tick(Engine& e, const TickShape& sh, const float* features_dev, float* preds_dev,
                  hipStream_t s) {
   Group all;
-  all.r = Runs{e.d_slots, e.d_off, sh.n_runs, sh.n_rows, sh.steps, e.d_pos, e.d_rslot,
-               sh.n_long};
+  all.r = all_runs(e, sh);
   all.act_dev = e.d_act;
   all.act = sh.act;
   HK_TRY(stage_features(features_dev, sh.n_rows, e.d.F, e.d.Fpad, e.FE.f, e.FE.l, e.lp_fmt, s));
@@ -1290,13 +1315,10 @@ int enqueue_tick(Engine& e, const TickShape& sh, const float* features_dev, floa
   const bool split = sh.split < sh.n_runs;
   Group g1, g2;
   if (split) {
-    g1.r = Runs{e.d_slots, e.d_off, sh.split, sh.row_split, sh.steps, e.d_pos, e.d_rslot,
-                std::min(sh.n_long, sh.split)};
+    g1.r = group1_runs(e, sh);
     g1.act_dev = e.d_act1;
     g1.act = sh.act1;
-    g2.r = Runs{e.d_slots + sh.split, e.d_off2, sh.n_runs - sh.split, sh.n_rows - sh.row_split,
-                sh.steps2, e.d_pos + sh.row_split, e.d_rslot + sh.row_split,
-                std::max(sh.n_long - sh.split, 0)};
+    g2.r = group2_runs(e, sh);
     g2.act_dev = e.d_act2;
     g2.act = sh.act2;
     g2.row0 = sh.row_split;
@@ -1933,11 +1955,8 @@ int hk_engine_tick(void* h, const int* slot_ids_host, const int* run_off_host, i
   const int k = e.stage_idx;
   e.stage_idx ^= 1;
   HK_CHECK_HIP(hipEventSynchronize(e.stage_done[k]));
-  const int steps = run_off_host[1] - run_off_host[0];
-  // xLSTM run groups: runs [0, split) and [split, n_runs).
-  const int split = hk::xlstm_split_point(run_off_host, n_runs, e.x_weight_us);
-  const int row_split = run_off_host[split];
-  const int steps2 = split < n_runs ? run_off_host[split + 1] - run_off_host[split] : 0;
+  hk::TickShape sh = hk::tick_shape(e, run_off_host, n_runs);
+  const int steps = sh.steps, split = sh.split, row_split = sh.row_split, steps2 = sh.steps2;
   int* stage = e.h_stage + (size_t)k * e.stage_ints();
   int* h_slots = stage;
   int* h_off = h_slots + e.max_runs;
@@ -1968,16 +1987,6 @@ int hk_engine_tick(void* h, const int* slot_ids_host, const int* run_off_host, i
                               s));
   HK_CHECK_HIP(hipEventRecord(e.stage_done[k], s));
 
-  hk::TickShape sh;
-  sh.n_runs = n_runs;
-  sh.n_rows = n_rows;
-  sh.steps = steps;
-  sh.split = split;
-  sh.row_split = row_split;
-  sh.steps2 = steps2;
-  while (sh.n_long < n_runs &&
-         run_off_host[sh.n_long + 1] - run_off_host[sh.n_long] > hk::kLogCapMax)
-    ++sh.n_long;
   sh.act.assign(h_act, h_act + steps);
   sh.act1.assign(h_act1, h_act1 + steps);
   sh.act2.assign(h_act2, h_act2 + steps2);
@@ -2006,6 +2015,29 @@ int hk_engine_graphs(void* h, int max_rows, int max_graphs) {
         if (x) HK_CHECK_HIP(hipGraphExecDestroy(x));
     e.graphs.clear();
   }
+  return HK_OK;
+}
+
+int hk_engine_tick_route(void* h, const int* run_off_host, int n_runs, int* route) {
+  HK_REQUIRE(h && run_off_host && route, "hk_engine_tick_route: null argument");
+  const Engine& e = *static_cast<Engine*>(h);
+  HK_REQUIRE(n_runs >= 1 && run_off_host[0] == 0, "hk_engine_tick_route: no runs");
+  for (int i = 0; i < n_runs; ++i) {
+    const int len = run_off_host[i + 1] - run_off_host[i];
+    HK_REQUIRE(len >= 1 && (i == 0 || len <= run_off_host[i] - run_off_host[i - 1]),
+               "hk_engine_tick_route: runs must be sorted by non-increasing length");
+  }
+  const hk::TickShape sh = hk::tick_shape(e, run_off_host, n_runs);
+  auto streamed = [&](int tower, const hk::Runs& r) {
+    const hk::MatScanDesc m = hk::run_scan_desc(e, tower, 0, r);
+    return r.n_runs > 0 && hk::stream_scan_takes(m) ? r.n_runs - r.n_long : 0;
+  };
+  const bool split = sh.split < n_runs;
+  route[0] = sh.split;
+  route[1] = streamed(hk::kXLSTM, split ? hk::group1_runs(e, sh) : hk::all_runs(e, sh));
+  route[2] = split ? streamed(hk::kXLSTM, hk::group2_runs(e, sh)) : 0;
+  route[3] = streamed(hk::kMamba2, hk::all_runs(e, sh));
+  route[4] = streamed(hk::kRetNet, hk::all_runs(e, sh));
   return HK_OK;
 }
 

@@ -40,6 +40,7 @@ _lib.register("hk_engine_tick", c_int, [c_void_p, c_void_p, c_void_p, c_int, c_v
 
 _lib.register("hk_engine_check", c_int, [c_void_p, c_void_p])
 _lib.register("hk_engine_graphs", c_int, [c_void_p, c_int, c_int])
+_lib.register("hk_engine_tick_route", c_int, [c_void_p, c_void_p, c_int, c_void_p])
 _lib.register("hk_engine_graph_info", c_int, [c_void_p] + [ctypes.POINTER(c_int64)] * 3)
 _lib.register("hk_engine_profile", c_int, [c_void_p, c_int])
 _lib.register("hk_engine_profile_read", c_int, [c_void_p, c_int, ctypes.POINTER(c_int), ctypes.POINTER(ctypes.c_double)])
@@ -404,6 +405,17 @@ class Engine:
         _lib.check(_lib.lib().hk_engine_graph_info(self._h, *[ctypes.byref(v) for v in vals]),
                    "hk_engine_graph_info")
         return dict(zip(("cached", "captures", "replays"), (v.value for v in vals)))
+
+    def tick_route(self, lengths) -> dict:
+        """How a tick of runs of these lengths (longest first) would be
+        scheduled: "split", the first run of the second xLSTM group
+        (len(lengths): one group), and the runs whose matrix-state scan streams
+        the tiles, "xlstm1", "xlstm2", "mamba2" and "retnet". Nothing runs."""
+        off = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+        out = np.zeros(5, np.int32)
+        _lib.check(_lib.lib().hk_engine_tick_route(self._h, off.ctypes.data, len(off) - 1, out.ctypes.data),
+                   "hk_engine_tick_route")
+        return dict(zip(("split", "xlstm1", "xlstm2", "mamba2", "retnet"), out.tolist()))
 
     def check(self):
         """Wait for the current stream's work (every tick enqueued on it) and

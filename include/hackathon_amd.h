@@ -294,6 +294,13 @@ int hk_engine_graphs(void* handle, int max_rows, int max_graphs);
  * counterpart (test and measurement support). */
 int hk_engine_graph_info(void* handle, int64_t* cached, int64_t* captures, int64_t* replays);
 
+/* How a tick of these length-sorted runs would be scheduled: route[0] the
+ * first run of the second xLSTM group (n_runs: one group), route[1 .. 4] the
+ * runs whose matrix-state scan streams the tiles, of the first xLSTM group,
+ * the second, Mamba2 and RetNet. Nothing is enqueued. No reference
+ * counterpart (test and measurement support). */
+int hk_engine_tick_route(void* handle, const int* run_off_host, int n_runs, int* route);
+
 /* Waits for the work enqueued on `stream` (a tick's stream: every tick joins
  * its side streams back into it, so this covers whole ticks; other work on
  * the device is not waited for); returns -2 if a persistent kernel's step

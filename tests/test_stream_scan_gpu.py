@@ -1,9 +1,10 @@
 """The streaming matrix scan (launches of many short runs over 256-column
 tiles) through whole ticks against the oracle's rounds in fp32: every run
 length it dispatches on (1, 2, 3-4, 5-8), logs from empty to full so that
-tiles are kept, written back and emptied, and a launch whose few long runs go
-to the general scan first. One run fewer than the rule asks for takes the
-general scan and agrees as well.
+tiles are kept, written back and emptied, a launch whose few long runs go to
+the general scan first, and the second xLSTM group of a split tick whose first
+keeps the general scan. One run fewer than the rule asks for takes the general
+scan and agrees as well. Engine.tick_route says which scan each launch took.
 
 Bound, per tower: the engine's distance from the float64 rounds (2-norm over
 all predictions) within twice that of the reference's own fp32 rounds, as for
@@ -25,6 +26,9 @@ pytestmark = pytest.mark.gpu
 # mLSTM heads of 256: eight 256 x 256 tiles per run, so 64 runs are the 512
 # work-groups the rule asks for
 CFG = spec.ModelConfig(hidden_size=1024, proj_size=256, tower_depth=1, num_heads=8, num_features=7)
+# RetNet heads of 256, which no long run below sixteen steps splits by rows: a
+# launch of both kinds of runs
+CFG4 = spec.ModelConfig(hidden_size=1024, proj_size=256, tower_depth=1, num_heads=4, num_features=7)
 SHORT = [8] * 3 + [7, 5] + [4] * 3 + [3] * 2 + [2] * 6
 
 
@@ -33,15 +37,21 @@ def params():
     return weights.generate(CFG, 0)
 
 
-@pytest.mark.parametrize("lens", [SHORT + [1] * (64 - len(SHORT)), SHORT + [1] * (63 - len(SHORT)),
-                                  [19, 9] + SHORT + [1] * (256 - len(SHORT))],
-                         ids=["64 runs", "63 runs", "two long"])
-def test_ticks_match_reference_rounds(dev, params, lens):
+@pytest.mark.parametrize("cfg,lens,routes", [
+    (CFG, SHORT + [1] * (64 - len(SHORT)), {"split": 64, "xlstm1": 64, "retnet": 0}),
+    (CFG, SHORT + [1] * (63 - len(SHORT)), {"split": 63, "xlstm1": 0, "retnet": 0}),
+    (CFG, [19, 9] + SHORT + [1] * (256 - len(SHORT)), {"split": 124, "xlstm1": 0, "xlstm2": 134}),
+    (CFG4, [12, 9] + SHORT + [1] * (256 - len(SHORT)), {"retnet": 256, "xlstm1": 0}),
+], ids=["64 runs", "63 runs", "second group", "two long"])
+def test_ticks_match_reference_rounds(dev, params, cfg, lens, routes):
     from hackathon_amd.engine import Engine, pack_runs
 
     n = len(lens)
-    eng = Engine(CFG, capacity=n, max_rows=sum(lens), linear_dtype="fp32")
+    params = params if cfg is CFG else weights.generate(cfg, 0)
+    eng = Engine(cfg, capacity=n, max_rows=sum(lens), linear_dtype="fp32")
     eng.load_weights(params)
+    got = eng.tick_route(lens)
+    assert {k: got[k] for k in routes} == routes
     rng = np.random.default_rng(n)
     hist, got = [[] for _ in range(n)], [[] for _ in range(n)]
     for tick in range(3):
@@ -49,7 +59,7 @@ def test_ticks_match_reference_rounds(dev, params, lens):
         # meet runs of every length
         syms = np.roll(np.arange(n), 5 * tick).astype(np.int32)
         runs, order = pack_runs(syms, np.asarray(lens))
-        x = np.clip(rng.standard_normal((sum(lens), CFG.num_features)), -5, 5).astype(np.float32)
+        x = np.clip(rng.standard_normal((sum(lens), cfg.num_features)), -5, 5).astype(np.float32)
         preds = eng.tick(runs, torch.from_numpy(x).to(dev)).cpu().numpy()
         for pos, i in enumerate(order):
             a, b = int(runs.run_off[pos]), int(runs.run_off[pos + 1])
@@ -57,8 +67,8 @@ def test_ticks_match_reference_rounds(dev, params, lens):
             got[syms[i]].extend(preds[a:b])
     eng.check()
     eng.close()
-    p32, _ = reference_rounds(om.Params(params), CFG, hist)
-    p64, _ = reference_rounds(om.Params(params, dtype=torch.float64), CFG, hist)
+    p32, _ = reference_rounds(om.Params(params), cfg, hist)
+    p64, _ = reference_rounds(om.Params(params, dtype=torch.float64), cfg, hist)
     cat = lambda v: np.concatenate([np.asarray(a, np.float64) for a in v])
     g, w32, w64 = cat(got), cat(p32), cat(p64)
     err, ref = (np.linalg.norm(v - w64, axis=0) for v in (g, w32))
@@ -74,12 +84,13 @@ def test_a_bad_request_leaves_the_earlier_answers(dev, params, dtype, bad):
     written back)."""
     from hackathon_amd.engine import Engine, Runs
 
-    lens = sorted(SHORT + [1] * (64 - len(SHORT)), reverse=True)
+    lens = SHORT + [1] * (64 - len(SHORT))
     n, rows = len(lens), sum(lens)
     off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     last = off[1:] - 1
     eng = Engine(CFG, capacity=2 * n, max_rows=rows, linear_dtype=dtype)
     eng.load_weights(params)
+    assert eng.tick_route(lens)["xlstm1"] == n
     rng = np.random.default_rng(1)
     x = lambda: np.clip(rng.standard_normal((rows, CFG.num_features)), -5, 5).astype(np.float32)
     tick = lambda slot0, f: eng.tick(Runs(np.arange(slot0, slot0 + n, dtype=np.int32), off),
