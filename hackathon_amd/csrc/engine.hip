@@ -1294,10 +1294,23 @@ Runs group1_runs(const Engine& e, const TickShape& sh) {
   return Runs{e.d_slots, e.d_off, sh.split, sh.row_split, sh.steps, e.d_pos, e.d_rslot,
               std::min(sh.n_long, sh.split)};
 }
+// A second xLSTM group of fewer than kStreamBeside runs keeps its scans on the
+// general kernel (its count of long runs is given as not known). A small
+// group's streaming scan takes HBM from the first group's longer chain without
+// shortening the tick. Measured at the default widths, bf16, longest run 16,
+// 24 and 48, streaming / not, us:
+// - 64 runs (37 to 46 in the second group), two layers 1012 / 991, 1100 / 1075,
+//   1237 / 1213, twelve 5509 / 5378, 6000 / 5858, 6994 / 6971;
+// - 96 runs (53 to 62), two layers 1202 / 1205, 1276 / 1261, 1467 / 1436;
+// - 128 runs (69 to 78), two layers 1411 / 1453, 1493 / 1488, 1655 / 1643,
+//   twelve 7987 / 8325, 8438 / 8578, 9344 / 9267;
+// - 192 and 256 runs: streaming ahead by 1 to 7 %.
+constexpr int kStreamBeside = 64;
 Runs group2_runs(const Engine& e, const TickShape& sh) {
-  return Runs{e.d_slots + sh.split, e.d_off2, sh.n_runs - sh.split, sh.n_rows - sh.row_split,
-              sh.steps2, e.d_pos + sh.row_split, e.d_rslot + sh.row_split,
-              std::max(sh.n_long - sh.split, 0)};
+  const int n2 = sh.n_runs - sh.split;
+  return Runs{e.d_slots + sh.split, e.d_off2, n2, sh.n_rows - sh.row_split, sh.steps2,
+              e.d_pos + sh.row_split, e.d_rslot + sh.row_split,
+              n2 < kStreamBeside ? -1 : std::max(sh.n_long - sh.split, 0)};
 }
 
 // The device work of one tick on stream s, descriptors already in d_desc:
