@@ -530,19 +530,20 @@ def xlstm_layer_weight_us(cfg, lowp=True):
     return nbytes / 5.0e6
 
 
-def xlstm_split_point(run_off, weight_us=0.0):
+def xlstm_split_point(run_off, weight_us=0.0, lowp=True):
     """The engine's split of a tick's length-sorted runs into two xLSTM run
-    groups (engine.hip xlstm_split_point: 3 us per sLSTM step of a group's
-    longest run plus 5 us per symbol, a split charged one more read of a
-    layer's weights (weight_us), split when the larger group's cost plus
-    that read is under 0.8 of the whole), for ticks whose longest run has at
-    least 16 requests, as the replayed ticks have; the engine keeps ticks of
-    shorter runs whole below 192 runs. Returns the first run of the
-    second group (len(runs) for no split)."""
+    groups (engine.hip xlstm_split_point: whole below 192 runs whose longest
+    has fewer than 9 requests, or 16 with fp32 linears (lowp False); else 3 us
+    per sLSTM step of a group's longest run plus 5 us per symbol, a split
+    charged one more read of a layer's weights (weight_us), split when the
+    larger group's cost plus that read is under 0.8 of the whole). Returns the
+    first run of the second group (len(runs) for no split)."""
     n = len(run_off) - 1
     if n < 2:
         return n
     lens = np.diff(run_off)
+    if lens[0] < (9 if lowp else 16) and n < 192:
+        return n
     whole = 3.0 * lens[0] + 5.0 * n
     best, best_k = whole, n
     for k in range(1, n):

@@ -1232,20 +1232,33 @@ int run_towers_mt(Engine& e, const Group& all, const Group& g1, const Group* g2,
 // bf16 (C4): about 1000 against 500 + 24.)
 // The second group also takes the stream that Hawk would have, so it has to
 // shorten a long chain of sLSTM steps: ticks whose longest run is below
-// kSplitMinLen stay whole (until they have very many runs, below). Two-layer ticks, us split / whole: 32, 64 and 256
-// single requests 685 / 637, 888 / 873 and 2349 / 2285; 256 with runs of up
-// to about six 2011 / 1968; 64 single requests in fp32 1309 / 1167; with a
-// run of about fifty 256 requests 1500 / 1574 and 800 3347 / 3629. From
-// kSplitMinRuns runs up two groups pay again: one group's scan reads HBM while
-// the other's projections keep the matrix cores busy (whole / split, back to back: 256
-// runs 2220 / 2147 us, 512 4130 / 3990, 610 5690 / 5365; 128 runs 1358 / 1492).
-constexpr int kSplitMinLen = 16;
+// kSplitMinLen stay whole, until kSplitMinRuns runs, where two groups pay for
+// any lengths (one group's scan reads HBM while the other's projections keep
+// the matrix cores busy).
+// - With 16-bit linears the line lies above the runs that fit the write-back
+//   log, whose scans stream in a whole tick. Default widths, whole / split, us,
+//   twelve layers: longest run 8 of 24, 64, 96 and 128 runs 3450 / 3516, 5102 /
+//   5118, 6326 / 6533 and 7787 / 7937; 10 of 48, 64, 96 and 128 runs 4758 /
+//   4505, 5456 / 5241, 6760 / 6551 and 8320 / 7954; 14 of 32, 64 and 128 runs
+//   4168 / 4098, 5676 / 5502 and 8566 / 8136 (10 to 14 of 24 runs within 1 %).
+//   Two layers: longest 10, 64 runs 978 / 992, 96 runs 1200 / 1246, 128 runs
+//   1455 / 1457.
+// - With fp32 linears a second read of the weights costs twice as much and the
+//   line lies higher. Twelve layers: longest run 9 and 14 of 32 runs 5521 / 6110
+//   and 5816 / 6361, of 64 runs 8669 / 8840 and 8863 / 9038, 14 of 128 runs 13777
+//   / 13643. Two layers, longest 14 of 32, 64 and 128 runs 1056 / 1191, 1602 /
+//   1678 and 2464 / 2483.
+// - Single requests, 16-bit, whole / split: 128 runs 7086 / 7126, 160 runs 8575 /
+//   8324, 176 runs 9240 / 8999, 192 runs 9724 / 9412, 256 runs 12161 / 11774 (two
+//   layers 1281 / 1317, 1550 / 1540, 1665 / 1653, 1756 / 1725, 2205 / 2134).
+constexpr int kSplitMinLenLp = kLogCapMax + 1;
+constexpr int kSplitMinLenF32 = 16;
 constexpr int kSplitMinRuns = 192;
-int xlstm_split_point(const int* run_off, int n_runs, double weight_us) {
+int xlstm_split_point(const int* run_off, int n_runs, double weight_us, bool lowp) {
   constexpr double kStepUs = 3.0, kSymbolUs = 5.0, kGain = 0.8;
   if (n_runs < 2) return n_runs;
   const int len0 = run_off[1] - run_off[0];
-  if (len0 < kSplitMinLen && n_runs < kSplitMinRuns) return n_runs;
+  if (len0 < (lowp ? kSplitMinLenLp : kSplitMinLenF32) && n_runs < kSplitMinRuns) return n_runs;
   const double whole = kStepUs * len0 + kSymbolUs * n_runs;
   double best = whole;
   int best_k = n_runs;
@@ -1278,7 +1291,7 @@ TickShape tick_shape(const Engine& e, const int* run_off, int n_runs) {
   sh.n_rows = run_off[n_runs];
   sh.steps = run_off[1] - run_off[0];
   // xLSTM run groups: runs [0, split) and [split, n_runs).
-  sh.split = xlstm_split_point(run_off, n_runs, e.x_weight_us);
+  sh.split = xlstm_split_point(run_off, n_runs, e.x_weight_us, e.lowp);
   sh.row_split = run_off[sh.split];
   sh.steps2 = sh.split < n_runs ? run_off[sh.split + 1] - run_off[sh.split] : 0;
   while (sh.n_long < n_runs && run_off[sh.n_long + 1] - run_off[sh.n_long] > kLogCapMax)

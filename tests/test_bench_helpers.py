@@ -64,14 +64,22 @@ def test_log_occupancy_is_bounded_on_zipf_ticks():
 def test_xlstm_split_point_hand_cases():
     """The replica of the engine's xLSTM group split (bench.xlstm_split_point):
     per group 3 us per sLSTM step of its longest run plus 5 us per symbol, a
-    split charged one more read of a layer's weights."""
+    split charged one more read of a layer's weights, for ticks of long enough
+    or many enough runs. (test_tick_route_gpu.py compares it with the engine.)"""
     one_each = lambda n: np.arange(n + 1)  # n runs of one request
-    # four one-request symbols: 3 + 20 = 23 unsplit; two and two cost 13
-    assert bench.xlstm_split_point(one_each(4)) == 2
-    # ... plus a second fp32 weight read (41 us): 54 > 0.8 * 23, no split
-    assert bench.xlstm_split_point(one_each(4), 40.5) == 4
-    # 64 one-request symbols: 323 unsplit, 163 + 24 split at 32 < 258.4
-    assert bench.xlstm_split_point(one_each(64), 23.7) == 32
+    # short runs stay whole below 192 of them, whatever the model says
+    assert bench.xlstm_split_point(one_each(4)) == 4
+    assert bench.xlstm_split_point(one_each(64), 23.7) == 64
+    assert bench.xlstm_split_point(one_each(191), 23.7) == 191
+    # 192: 963 unsplit, 483 + 24 split at 96 < 770.4
+    assert bench.xlstm_split_point(one_each(192), 23.7) == 96
+    # a longest run of 8 and of 9 with 16-bit linears, of 15 and 16 with fp32
+    # (max(3 L + 5 k, 3 + 5 (64 - k)) is least at k = 30 for 9, first at 27 for 16)
+    head = lambda L: np.concatenate([[0], np.cumsum([L] + [1] * 63)])
+    assert bench.xlstm_split_point(head(8), 23.7) == 64
+    assert bench.xlstm_split_point(head(9), 23.7) == 30
+    assert bench.xlstm_split_point(head(15), 40.5, lowp=False) == 64
+    assert bench.xlstm_split_point(head(16), 40.5, lowp=False) == 27
     # a 40-request run and 100 single ones: max(120 + 5k, 3 + 5(101 - k))
     # is least at k = 39 (315 against 318 at k = 38 and 320 at k = 40)
     run_off = np.concatenate([[0], np.cumsum([40] + [1] * 100)])
