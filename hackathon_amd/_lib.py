@@ -105,11 +105,14 @@ def ptr(t) -> int:
 
 
 def current_stream(device) -> int:
-    """The raw handle of torch's current stream on a CUDA device. Taken from
-    the binding torch.cuda.current_stream wraps: every operator call asks for
-    it, and the Stream object costs the call about as much as its checks."""
+    """The raw handle of torch's current stream on a CUDA device (as
+    torch.cuda.current_stream takes it: a device, its name or its index). For
+    an indexed torch.device from the binding that torch.cuda.current_stream
+    wraps, where torch has it: every operator call asks for the stream, and
+    the Stream object costs the call about as much as its checks."""
     import torch
 
-    if device.index is None:
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None or not isinstance(device, torch.device) or device.index is None:
         return torch.cuda.current_stream(device).cuda_stream
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    return raw(device.index)

@@ -42,3 +42,23 @@ def test_python_binding_covers_header():
     lib = _lib.lib()
     assert lib.hk_version() >= 1
     assert isinstance(lib.hk_last_error(), bytes)
+
+
+@pytest.mark.parametrize("raw", [True, False])
+def test_current_stream_takes_what_torch_takes(monkeypatch, raw):
+    """_lib.current_stream on a device, its name, its index and a device
+    without an index, with and without torch's raw-handle binding (stubs: no
+    GPU here)."""
+    import torch
+    from types import SimpleNamespace
+
+    from hackathon_amd import _lib
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: SimpleNamespace(cuda_stream=41))
+    if raw:
+        monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda i: 42 + i, raising=False)
+    else:
+        monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    assert _lib.current_stream(torch.device("cuda:1")) == (43 if raw else 41)
+    for device in (torch.device("cuda"), "cuda:0", 0, None):
+        assert _lib.current_stream(device) == 41
