@@ -926,6 +926,10 @@ int round_lp_inplace(float* v, int64_t n, int lp_fmt, hipStream_t s) {
 }
 
 void CopyList::add(const float* s, float* d, int64_t floats) {
+  if (count >= kMax) {
+    count = kMax + 1;  // refused by copy_list
+    return;
+  }
   src[count] = s;
   dst[count] = d;
   n[count] = floats;
@@ -934,6 +938,7 @@ void CopyList::add(const float* s, float* d, int64_t floats) {
 }
 
 int copy_list(const CopyList& c, hipStream_t s) {
+  HK_REQUIRE(c.count <= CopyList::kMax, "copy_list: more than %d arrays", CopyList::kMax);
   const int64_t blocks = c.block0[c.count];
   if (blocks == 0) return HK_OK;
   HK_REQUIRE(blocks < (1LL << 31), "copy_list: too large (%lld work-groups)", (long long)blocks);
