@@ -335,6 +335,48 @@ int elementwise_grid(int64_t n, unsigned* blocks) {
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
+// The common part of the CastLinear entries `who`: g holds the operands, the
+// bias and the weight's layout. Workspace layout: kCastArrivals arrival
+// counters, then split-K partial sums. With rows, they are cast to format fmt
+// into rows_lp (= g.A) first.
+int cast_gemm(const char* who, GemmArgs& g, int M, int N, int K, int fmt, float* out,
+              void* workspace, int64_t workspace_bytes, hipStream_t s,
+              const float* rows = nullptr, uint16_t* rows_lp = nullptr) {
+  constexpr int64_t kCastArrivals = 1 << 16;
+  HK_REQUIRE(fmt == kLpBF16 || fmt == kLpF16, "%s: format %d", who, fmt);
+  HK_REQUIRE(aligned16(g.A) && aligned16(g.W), "%s: operands must be 16-byte aligned", who);
+  HK_REQUIRE(workspace == nullptr || workspace_bytes >= kCastArrivals * 4,
+             "%s: a workspace needs at least %lld bytes", who, (long long)kCastArrivals * 4);
+  if (M == 0) return HK_OK;
+  if (rows != nullptr) {
+    const int64_t n = (int64_t)M * K;
+    const unsigned blocks = (unsigned)std::min<int64_t>((n / 8 + 255) / 256, 2048);
+    if (fmt == kLpF16)
+      hipLaunchKernelGGL(cast_rows_kernel<kLpF16>, dim3(blocks), dim3(256), 0, s, rows, rows_lp, n);
+    else
+      hipLaunchKernelGGL(cast_rows_kernel<kLpBF16>, dim3(blocks), dim3(256), 0, s, rows, rows_lp, n);
+    HK_LAUNCH_CHECK();
+  }
+  g.type = fmt == kLpF16 ? GemmType::kF16 : GemmType::kBF16;
+  g.lda = K;
+  if (!g.w_packed) g.ldw = K;
+  g.M = M;
+  g.N = N;
+  g.K = K;
+  g.ep.round_lp = true;
+  g.ep.lp_fmt = fmt;
+  g.ep.out = out;
+  g.ep.ldo = N;
+  GemmWorkspace ws;
+  if (workspace != nullptr) {
+    ws.arrivals = static_cast<int*>(workspace);
+    ws.arrival_elems = kCastArrivals;
+    ws.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCastArrivals * 4);
+    ws.partial_elems = (workspace_bytes - kCastArrivals * 4) / 4;
+  }
+  return gemm(g, ws, s);
+}
+
 }  // namespace
 
 int hcontract_row_step(float* S, const float* alpha, int64_t alpha_head_stride,
@@ -357,10 +399,6 @@ int hcontract_row_step(float* S, const float* alpha, int64_t alpha_head_stride,
   HK_LAUNCH_CHECK();
   return HK_OK;
 }
-
-namespace {
-
-}  // namespace
 
 }  // namespace hk
 
@@ -544,42 +582,19 @@ int hk_block_linear(const float* x, const float* weight, const float* bias, floa
 }
 
 // CastLinear.forward on 16-bit operands: the engine's projection GEMM with
-// its CastLinear epilogue. Workspace layout: kCastArrivals arrival counters,
-// then split-K partial sums.
+// its CastLinear epilogue (cast_gemm).
 int hk_cast_linear(const uint16_t* x, const uint16_t* w, const float* bias, float* out, int M,
                    int N, int K, int fmt, void* workspace, int64_t workspace_bytes,
                    void* stream) {
-  constexpr int64_t kCastArrivals = 1 << 16;
   HK_REQUIRE(x && w && out, "hk_cast_linear: null operand");
   HK_REQUIRE(M >= 0 && N > 0 && K > 0 && K % 64 == 0,
              "hk_cast_linear: bad shape M=%d N=%d K=%d (K a multiple of 64)", M, N, K);
-  HK_REQUIRE(fmt == hk::kLpBF16 || fmt == hk::kLpF16, "hk_cast_linear: format %d", fmt);
-  HK_REQUIRE(hk::aligned16(x) && hk::aligned16(w), "hk_cast_linear: operands must be 16-byte aligned");
-  HK_REQUIRE(workspace == nullptr || workspace_bytes >= kCastArrivals * 4,
-             "hk_cast_linear: a workspace needs at least %lld bytes", (long long)kCastArrivals * 4);
-  if (M == 0) return HK_OK;
   hk::GemmArgs g;
-  g.type = fmt == hk::kLpF16 ? hk::GemmType::kF16 : hk::GemmType::kBF16;
   g.A = x;
-  g.lda = K;
   g.W = w;
-  g.ldw = K;
-  g.M = M;
-  g.N = N;
-  g.K = K;
   g.ep.bias = bias;
-  g.ep.round_lp = true;
-  g.ep.lp_fmt = fmt;
-  g.ep.out = out;
-  g.ep.ldo = N;
-  hk::GemmWorkspace ws;
-  if (workspace != nullptr) {
-    ws.arrivals = static_cast<int*>(workspace);
-    ws.arrival_elems = kCastArrivals;
-    ws.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCastArrivals * 4);
-    ws.partial_elems = (workspace_bytes - kCastArrivals * 4) / 4;
-  }
-  return hk::gemm(g, ws, (hipStream_t)stream);
+  return hk::cast_gemm("hk_cast_linear", g, M, N, K, fmt, out, workspace, workspace_bytes,
+                       (hipStream_t)stream);
 }
 
 int hk_pack_cast_weight(const uint16_t* w, uint16_t* packed, int N, int K, void* stream) {
@@ -589,94 +604,40 @@ int hk_pack_cast_weight(const uint16_t* w, uint16_t* packed, int N, int K, void*
 int hk_cast_linear_packed(const uint16_t* x, const uint16_t* w_packed, const float* bias,
                           float* out, int M, int N, int K, int fmt, int min_work_groups,
                           void* workspace, int64_t workspace_bytes, void* stream) {
-  constexpr int64_t kCastArrivals = 1 << 16;
   HK_REQUIRE(x && w_packed && out, "hk_cast_linear_packed: null operand");
   HK_REQUIRE(M >= 0 && hk::packable(N, K),
              "hk_cast_linear_packed: bad shape M=%d N=%d K=%d (N a multiple of 32, K of 64)", M,
              N, K);
-  HK_REQUIRE(fmt == hk::kLpBF16 || fmt == hk::kLpF16, "hk_cast_linear_packed: format %d", fmt);
-  HK_REQUIRE(hk::aligned16(x) && hk::aligned16(w_packed),
-             "hk_cast_linear_packed: operands must be 16-byte aligned");
   HK_REQUIRE(min_work_groups >= 0, "hk_cast_linear_packed: min_work_groups=%d", min_work_groups);
-  HK_REQUIRE(workspace == nullptr || workspace_bytes >= kCastArrivals * 4,
-             "hk_cast_linear_packed: a workspace needs at least %lld bytes",
-             (long long)kCastArrivals * 4);
-  if (M == 0) return HK_OK;
   hk::GemmArgs g;
-  g.type = fmt == hk::kLpF16 ? hk::GemmType::kF16 : hk::GemmType::kBF16;
   g.A = x;
-  g.lda = K;
   g.W = w_packed;
   g.w_packed = true;
   g.min_tiles = min_work_groups;
-  g.M = M;
-  g.N = N;
-  g.K = K;
   g.ep.bias = bias;
-  g.ep.round_lp = true;
-  g.ep.lp_fmt = fmt;
-  g.ep.out = out;
-  g.ep.ldo = N;
-  hk::GemmWorkspace ws;
-  if (workspace != nullptr) {
-    ws.arrivals = static_cast<int*>(workspace);
-    ws.arrival_elems = kCastArrivals;
-    ws.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCastArrivals * 4);
-    ws.partial_elems = (workspace_bytes - kCastArrivals * 4) / 4;
-  }
-  return hk::gemm(g, ws, (hipStream_t)stream);
+  return hk::cast_gemm("hk_cast_linear_packed", g, M, N, K, fmt, out, workspace, workspace_bytes,
+                       (hipStream_t)stream);
 }
 
 int hk_cast_linear_f32(const float* x, uint16_t* x_lp, const uint16_t* w, const uint16_t* bias,
                        float* out, int M, int N, int K, int fmt, int packed, int min_work_groups,
                        void* workspace, int64_t workspace_bytes, void* stream) {
-  constexpr int64_t kCastArrivals = 1 << 16;
   HK_REQUIRE(x && x_lp && w && out, "hk_cast_linear_f32: null operand");
   HK_REQUIRE(M >= 0 && N > 0 && K > 0 && K % 64 == 0,
              "hk_cast_linear_f32: bad shape M=%d N=%d K=%d (K a multiple of 64)", M, N, K);
   HK_REQUIRE(!packed || hk::packable(N, K),
              "hk_cast_linear_f32: bad packed shape N=%d K=%d (N a multiple of 32, K of 64)", N, K);
-  HK_REQUIRE(fmt == hk::kLpBF16 || fmt == hk::kLpF16, "hk_cast_linear_f32: format %d", fmt);
-  HK_REQUIRE(hk::aligned16(x) && hk::aligned16(x_lp) && hk::aligned16(w),
-             "hk_cast_linear_f32: operands must be 16-byte aligned");
+  HK_REQUIRE(hk::aligned16(x), "hk_cast_linear_f32: operands must be 16-byte aligned");
   HK_REQUIRE(min_work_groups >= 0, "hk_cast_linear_f32: min_work_groups=%d", min_work_groups);
-  HK_REQUIRE(workspace == nullptr || workspace_bytes >= kCastArrivals * 4,
-             "hk_cast_linear_f32: a workspace needs at least %lld bytes",
-             (long long)kCastArrivals * 4);
-  if (M == 0) return HK_OK;
-  hipStream_t s = (hipStream_t)stream;
-  const int64_t n = (int64_t)M * K;
-  const unsigned blocks = (unsigned)std::min<int64_t>((n / 8 + 255) / 256, 2048);
-  if (fmt == hk::kLpF16)
-    hipLaunchKernelGGL(hk::cast_rows_kernel<hk::kLpF16>, dim3(blocks), dim3(256), 0, s, x, x_lp, n);
-  else
-    hipLaunchKernelGGL(hk::cast_rows_kernel<hk::kLpBF16>, dim3(blocks), dim3(256), 0, s, x, x_lp, n);
-  HK_LAUNCH_CHECK();
   hk::GemmArgs g;
-  g.type = fmt == hk::kLpF16 ? hk::GemmType::kF16 : hk::GemmType::kBF16;
   g.A = x_lp;
-  g.lda = K;
   g.W = w;
-  g.ldw = K;
   g.w_packed = packed != 0;
   g.min_tiles = min_work_groups;
-  g.M = M;
-  g.N = N;
-  g.K = K;
   g.ep.bias = reinterpret_cast<const float*>(bias);
   g.ep.bias_lp = bias != nullptr;
-  g.ep.round_lp = true;
-  g.ep.lp_fmt = fmt;
-  g.ep.out = out;
-  g.ep.ldo = N;
-  hk::GemmWorkspace ws;
-  if (workspace != nullptr) {
-    ws.arrivals = static_cast<int*>(workspace);
-    ws.arrival_elems = kCastArrivals;
-    ws.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCastArrivals * 4);
-    ws.partial_elems = (workspace_bytes - kCastArrivals * 4) / 4;
-  }
-  return hk::gemm(g, ws, s);
+  return hk::cast_gemm("hk_cast_linear_f32", g, M, N, K, fmt, out, workspace, workspace_bytes,
+                       (hipStream_t)stream, x, x_lp);
 }
 
 int hk_rglru_step(float* h, const float* x, const float* gate_i, const float* gate_r,
