@@ -112,7 +112,9 @@ def current_stream(device) -> int:
     the Stream object costs the call about as much as its checks."""
     import torch
 
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is None or not isinstance(device, torch.device) or device.index is None:
-        return torch.cuda.current_stream(device).cuda_stream
-    return raw(device.index)
+    if isinstance(device, torch.device) and (index := device.index) is not None:
+        try:
+            return torch._C._cuda_getCurrentRawStream(index)
+        except AttributeError:  # a torch without the binding
+            pass
+    return torch.cuda.current_stream(device).cuda_stream
