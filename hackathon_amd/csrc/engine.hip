@@ -1307,23 +1307,31 @@ Runs group1_runs(const Engine& e, const TickShape& sh) {
   return Runs{e.d_slots, e.d_off, sh.split, sh.row_split, sh.steps, e.d_pos, e.d_rslot,
               std::min(sh.n_long, sh.split)};
 }
-// A second xLSTM group of fewer than kStreamBeside runs keeps its scans on the
-// general kernel (its count of long runs is given as not known). A small
-// group's streaming scan takes HBM from the first group's longer chain without
-// shortening the tick. Measured at the default widths, bf16, longest run 16,
-// 24 and 48, streaming / not, us:
-// - 64 runs (37 to 46 in the second group), two layers 1012 / 991, 1100 / 1075,
-//   1237 / 1213, twelve 5509 / 5378, 6000 / 5858, 6994 / 6971;
-// - 96 runs (53 to 62), two layers 1202 / 1205, 1276 / 1261, 1467 / 1436;
-// - 128 runs (69 to 78), two layers 1411 / 1453, 1493 / 1488, 1655 / 1643,
-//   twelve 7987 / 8325, 8438 / 8578, 9344 / 9267;
-// - 192 and 256 runs: streaming ahead by 1 to 7 %.
+// A second xLSTM group streams its matrix states only from kStreamBeside runs
+// and from kStreamSlack more runs than the tick has steps; a smaller one keeps
+// the general scan (its count of long runs is given as not known). Its stream of
+// tiles takes HBM from the first group's chain, the more the longer that chain,
+// and has to be long itself to gain. Measured at the default widths in bf16,
+// twelve layers, streaming / not, us (steps, runs in the second group):
+// - 16 steps: 37 runs 5509 / 5378, 65 runs 7698 / 7902, 93 runs 9801 / 10432;
+// - 24 and 32: 39 runs 6000 / 5858, 67 runs 7961 / 8164, 69 runs 8227 / 8342;
+// - 40 and 48: 76 runs 8982 / 8964, 74 runs 9023 / 8921, 82 runs 9636 / 9757;
+// - Zipf ticks: 42 steps, 66 runs 8720 / 8360 (the headline tick, 46 steps and
+//   about 70 runs, 8.61 / 8.44 ms); 53 steps, 80 runs 10130 / 9980, 103 runs
+//   12025 / 12295; 69 steps, 94 runs 11700 / 11480; 80 steps, 115 runs 14170 /
+//   14280; 96 steps, 171 runs 20280 / 21150; 136 steps, 100 runs 14250 / 13980,
+//   207 runs 25170 / 26010.
+// (Two layers give the same signs: 16 steps, 37 runs 1012 / 991, 69 runs 1411 /
+// 1453; 42 steps, 66 runs 1547 / 1514; 115 steps, 84 runs 2037 / 1938.)
 constexpr int kStreamBeside = 64;
+constexpr int kStreamSlack = 32;
 Runs group2_runs(const Engine& e, const TickShape& sh) {
   const int n2 = sh.n_runs - sh.split;
   return Runs{e.d_slots + sh.split, e.d_off2, n2, sh.n_rows - sh.row_split, sh.steps2,
               e.d_pos + sh.row_split, e.d_rslot + sh.row_split,
-              n2 < kStreamBeside ? -1 : std::max(sh.n_long - sh.split, 0)};
+              n2 < std::max(kStreamBeside, sh.steps + kStreamSlack)
+                  ? -1
+                  : std::max(sh.n_long - sh.split, 0)};
 }
 
 // The device work of one tick on stream s, descriptors already in d_desc:

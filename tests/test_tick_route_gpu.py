@@ -22,17 +22,22 @@ def engine(request, dev):
     eng.close()
 
 
-def test_small_second_group_keeps_the_general_scan(engine):
-    """The second group of a split tick streams its tiles from 64 runs up (at
-    eight heads of 512 columns 32 runs fill the device)."""
+@pytest.mark.parametrize("steps,line", [(24, 64), (32, 64), (48, 80)])
+def test_small_second_group_keeps_the_general_scan(engine, steps, line):
+    """The second group of a split tick streams its tiles from 64 runs up, and
+    from 32 more runs than the tick has steps (at eight heads of 512 columns 32
+    runs fill the device)."""
     seen = {}
-    for n in range(40, 160):
-        r = engine.tick_route([24] + [1] * (n - 1))
+    for n in range(40, 220):
+        r = engine.tick_route([steps] + [1] * (n - 1))
         if r["split"] < n:
             seen[n - r["split"]] = r["xlstm2"]
-    assert seen[63] == 0 and seen[40] == 0
-    assert seen[64] == 64 and seen[70] == 70
-    # one group: from 32 runs up
+    assert seen[line - 1] == 0 and seen[line - 10] == 0
+    assert seen[line] == line and seen[line + 6] == line + 6
+
+
+def test_one_group_streams_from_32_runs(engine):
+    """(2 x 8 x 32 work-groups of 256 columns.)"""
     assert engine.tick_route([1] * 31)["xlstm1"] == 0
     assert engine.tick_route([8] + [1] * 31)["xlstm1"] == 32
 
