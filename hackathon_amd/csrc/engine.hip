@@ -431,8 +431,14 @@ struct Engine {
   // runs), side[0] its second group, side[1] Mamba2, side[2] RetNet and
   // Hawk; a tick without a second group runs Hawk on side[0] (RetNet and
   // Hawk together are 42 of a two-layer tick's launches against the xLSTM's
-  // 32, and a small tick is the longest stream's chain of launches:
-  // 8 of 64 rows 642 us on one stream, 547 on two).
+  // 32, and a small tick is the longest stream's chain of launches). Single
+  // requests at the default widths, Hawk behind RetNet / on side[0], us, one
+  // tick at a time: two layers, bf16, 1, 16, 32 and 64 rows 395 / 371, 525 / 505,
+  // 673 / 619, 877 / 837; twelve layers, fp32, 2682 / 2563, 3609 / 3511, 5115 /
+  // 4834, 6446 / 6239; bf16 1706 / 1775, 2455 / 2477, 3256 / 3165, 4508 / 4525
+  // (back to back 1805 / 1907, 2549 / 2639, 3332 / 3265, 4543 / 4632): at full
+  // depth with 16-bit weights the xLSTM's chain is the longest either way and
+  // the smallest ticks lose what the third stream beside it costs.
   static constexpr int kSide = 3;
   hipStream_t side[kSide] = {nullptr, nullptr, nullptr};
   // hipGraph replay of small ticks (the reference captures its whole step

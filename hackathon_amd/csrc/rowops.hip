@@ -883,7 +883,10 @@ int mlstm_qkv_if(const ConvIn& conv, const float* x_m, int64_t ld_xm, const floa
   // Sixteen gate rows of few request rows go four to a work-group: one
   // work-group reads 12 KB of gate weights per 4-column block and would take
   // a segment's 196 KB through one CU (one row: 14.4 us, dealt out 10.5). From 64
-  // rows up (64 work-groups) the repeated q, k, v products cost more.
+  // rows up (64 work-groups) that gains nothing. Two-layer ticks of single
+  // requests, default widths, dealt out / not, us: 1 row 370 / 383, 8 rows 431 /
+  // 444, 32 rows 612 / 623, 48 rows 730 / 736, 63 rows 838 / 846, 64 rows 834 /
+  // 840, 80 rows 958 / 961.
   const dim3 block(256);
 #define HK_QKV_IF(NOUT, R)                                                                      \
   hipLaunchKernelGGL((mlstm_qkv_if_kernel<NOUT, R>), dim3(segs, (n_rows + (R)-1) / (R), n_out / (NOUT)), block, \

@@ -21,9 +21,16 @@
 // 256-column tile and streams them one 1 KB row per load, U at a time and two
 // such groups in flight; w_t (and b_j where the tile is written) come from
 // LDS, four rows per 16-byte read. The waves' sums meet in LDS once per run.
-// Measured alone (microseconds, this / mat_scan_kernel): 300 runs of 8
-// 512x512 tiles 483 / 528 (5.2 TB/s, what a large copy reaches on this card),
-// 64 runs 103 / 115; 300 runs of 8 256x256 tiles 134 / 149.
+// Measured alone (microseconds, this / mat_scan_kernel; runs of 1, 2, 4 and 8
+// steps, logs 0 to 5 entries full, so that most stay, then all full, so that
+// every tile is written):
+// - 300 runs of 8 512x512 tiles 438 / 480, 488 / 544, 619 / 653, 938 / 1031 (5.8
+//   TB/s read at one step); written 1002 / 1046, 1008 / 1071, 1020 / 1114, 1055 /
+//   1275 (5.0 TB/s);
+// - 64 runs 101 / 114, 111 / 125, 153 / 156, 216 / 249; written 226 / 244 to 252
+//   / 305;
+// - 300 runs of 8 256x256 tiles 125 / 139, 136 / 158, 183 / 204, 289 / 346;
+//   written 272 / 270, 276 / 282, 290 / 310, 339 / 377.
 #include <cstdint>
 
 #include "scan_mat.h"
@@ -414,13 +421,22 @@ __global__ __launch_bounds__(512, 4) void stream_scan_kernel(MatScanDesc d) {
 
 }  // namespace
 
-// Where the line lies: below 512 work-groups (two per CU) the tile moves in
-// fewer, longer pieces than mat_scan_kernel's and gains nothing (one to 32
-// runs 8.4 to 54 against 9.9 to 63 us alone, but no faster inside a tick).
-// Runs of more than eight steps go to mat_scan_kernel in a launch before this
-// one, which costs more than it gives until the short runs are many (a tick of
-// 85 runs, six of them long: 8.4 ms with two launches, 7.8 with one). Narrower
-// tiles (Mamba2's 128 x 64) read no faster this way (300 runs 151 / 142 us).
+// Where the lines lie (ticks of equal runs, default widths, bf16, two layers,
+// us, streaming / general; 512 work-groups are 32 runs of the mLSTM, 64 of
+// RetNet):
+// - From 512 work-groups, two per CU: 32 runs of 1, 4 and 8 steps 657 / 671, 812 /
+//   838, 1042 / 1106; 64 runs 845 / 880, 1203 / 1269, 1658 / 1823; 96 runs of 8
+//   2378 / 2593 (twelve layers, 64 runs 4688 / 4913, 6682 / 7043, 9593 / 10551).
+//   Below, in ticks of equal runs, it is ahead as well (24 runs of 1 and 8 steps
+//   568 / 579, 898 / 938): the line is on the safe side. The engine keeps the
+//   second xLSTM group of a split tick off it longer (group2_runs).
+// - Runs of more than eight steps go to mat_scan_kernel in a launch before this
+//   one. Taken from 256 short runs: 256 single runs beside two long ones 2336 /
+//   2447, 512 4152 / 4329. On the safe side too: streaming 192 would give 1855
+//   against 1975, 64 none (twelve layers, 64 and 96 runs 5406 / 5349 and 6699 /
+//   6588).
+// - Narrower tiles (Mamba2's 128 x 64) read no faster this way (300 runs 151 / 142
+//   us alone).
 bool stream_scan_takes(const MatScanDesc& d) {
   const int n_short = d.n_runs - d.n_long;
   return d.n_long >= 0 && !d.per_row && d.log_cap == kLogCapMax && d.row_parts == 1 &&

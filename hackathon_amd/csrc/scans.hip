@@ -807,8 +807,9 @@ __global__ void slstm_final_kernel(const int* __restrict__ slot_ids,
 //    wave sum per step would take 6 dependent shuffles each), and the waves'
 //    sums meet in LDS.
 // The rows of the next two blocks are prefetched into a register double
-// buffer; loads are unconditional (rows clamped to the run) so that the
-// compiler's wait counts stay exact.
+// buffer, rows clamped to the run instead of predicated, so that the compiler's
+// wait counts stay exact within a fill. Only runs of more than one block issue
+// the second fill (the wait behind that branch may be the longer one).
 constexpr int kGateBlock = 8;
 template <int NWV, int PER>
 __global__ __launch_bounds__(64 * NWV) void mlstm_gates_kernel(
