@@ -41,7 +41,7 @@ def params():
     (CFG, SHORT + [1] * (64 - len(SHORT)), {"split": 64, "xlstm1": 64, "retnet": 0}),
     (CFG, SHORT + [1] * (63 - len(SHORT)), {"split": 63, "xlstm1": 0, "retnet": 0}),
     (CFG, [19, 9] + SHORT + [1] * (256 - len(SHORT)), {"split": 124, "xlstm1": 0, "xlstm2": 134}),
-    (CFG4, [12, 9] + SHORT + [1] * (256 - len(SHORT)), {"retnet": 256, "xlstm1": 0}),
+    (CFG4, [12, 9] + SHORT + [1] * (256 - len(SHORT)), {"split": 126, "retnet": 256, "xlstm1": 0}),
 ], ids=["64 runs", "63 runs", "second group", "two long"])
 def test_ticks_match_reference_rounds(dev, params, cfg, lens, routes):
     from hackathon_amd.engine import Engine, pack_runs
